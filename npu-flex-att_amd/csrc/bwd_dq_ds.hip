@@ -134,6 +134,21 @@ void bwd_dq_ds_kernel(BwdArgs a) {
         g_hi = max(g_hi, hi);
       }
     }
+  // Interval masks: only the units the dK/dV kernel walked (and stored) are
+  // read: per query tile a range of KV blocks, non-decreasing in the tile.
+  auto doc_sub = [&](int t, int& lo, int& hi) {
+    int l, r;
+    ds_doc_range(p, b, t, nkb, l, r);
+    lo = SPU * l;
+    hi = min(SPU * r, nsb);
+  };
+  if (p.docc) {
+    int l, r, x;
+    doc_sub(qb * nq, l, x);
+    doc_sub(min(qb * nq + nq, nqt) - 1, x, r);
+    g_lo = __builtin_amdgcn_readfirstlane(max(g_lo, l));
+    g_hi = __builtin_amdgcn_readfirstlane(min(g_hi, r));
+  }
   const int nsub = g_hi > g_lo ? g_hi - g_lo : 0;
 
   // This wave's slots.
@@ -148,6 +163,20 @@ void bwd_dq_ds_kernel(BwdArgs a) {
       const int64_t unit = (int64_t)(b * p.Hq + hq_c[c]) * a.ds_head +
                            ds_tile_offset(t_c[c], p.causal, p.window, nkb);
       dsrc[c] = a.ds + unit * kDsUnitB + lane * 16;
+      if (p.docc) {
+        int l, r;
+        doc_sub(t_c[c], l, r);
+        l = __builtin_amdgcn_readfirstlane(max(l, s_lo[c]));
+        r = __builtin_amdgcn_readfirstlane(min(r, s_hi[c]));
+        if (r > l) {  // (l and the band's start are whole units)
+          dsrc[c] += (int64_t)((l - s_lo[c]) / SPU) * kDsUnitB;
+          s_lo[c] = l;
+          s_hi[c] = r;
+        } else {
+          dsrc[c] = (const char*)kp;
+          s_lo[c] = s_hi[c] = 0;
+        }
+      }
     } else {
       dsrc[c] = (const char*)kp;  // never used for data: a valid address to load from
     }

@@ -97,10 +97,15 @@ struct KvCfg {
 // PASS 0: dV and dK together; PASS 1: dV only; PASS 2: dK only (with the
 // staged dS when DS).  TPS: tiles per step (two: both phases of a step run
 // two consecutive tiles of the walk, 32 MFMAs per wave and phase, with one
-// exchange buffer; D = 128 without block maps).
+// exchange buffer; D = 128 without block maps).  DOC: interval masks narrow
+// the walk, in an instance of its own: the narrowing as a runtime branch cost
+// the plain kernels 0.6% (D = 128) and 1.3% (D = 256).  (The plain instances
+// never see column bounds, but keep the runtime form of the interval test
+// below: with constants in its place the D = 128 kernel's schedule is 2%
+// slower, 570 -> 580 us at bf16 B=2 Hq=32 Hkv=8 S=4096 causal.)
 // The tile stream of one work item: KV block kb of (b, hkv) = bh, walked as
 // workgroup slot `slot` (which sets the walk direction), in the LDS at smem.
-template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, int PASS, bool BLK, int TPS = 1>
+template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, int PASS, bool BLK, bool DOC, int TPS = 1>
 __device__ __forceinline__ void kv_tile_stream(const BwdArgs& a, char* smem, int slot, int kb, int bh) {
   using C = KvCfg<D, TPS>;
   static_assert(TPS == 1 || (TPS == 2 && PASS == 0 && !BLK && D == 128), "two tiles per step: D = 128, no block maps");
@@ -137,8 +142,20 @@ __device__ __forceinline__ void kv_tile_stream(const BwdArgs& a, char* smem, int
   int q_lo = 0, q_hi = p.Sq;
   if (p.causal) q_lo = n0;  // q >= kv >= n0
   if (p.window > 0) q_hi = min(q_hi, n0 + C::BKV + p.window);  // q - kv <= W
+  // The rows some key of the block may meet: packed documents of 700 keys on
+  // average at bf16 B=1 Hq=32 Hkv=8 S=8192 take 1107 -> 265 us here and 415 ->
+  // 110 us in dQ (the whole causal band was walked before).
+  if constexpr (DOC) {
+    int l, h;
+    kb_col_range(p, b, kb, l, h);
+    q_lo = __builtin_amdgcn_readfirstlane(max(q_lo, l));
+    q_hi = __builtin_amdgcn_readfirstlane(min(q_hi, h));
+  }
   const int qt_lo = q_lo / C::BM;
-  const int nqt = q_hi > q_lo ? (q_hi + C::BM - 1) / C::BM - qt_lo : 0;
+  // (interval masks: by whole tiles, as the dQ kernel counts them, ds_doc_range)
+  const int nqt = DOC            ? max((q_hi + C::BM - 1) / C::BM - qt_lo, 0)
+                  : q_hi > q_lo ? (q_hi + C::BM - 1) / C::BM - qt_lo
+                                : 0;
   int ntile = p.G * nqt;
   // Tile order: the G heads of a query tile consecutively; the first round
   // of workgroups (one per CU) walks the query tiles from the last one down,
@@ -964,7 +981,7 @@ __device__ __forceinline__ void kv_tile_stream(const BwdArgs& a, char* smem, int
 // D = 64 and 128 (PASS 0).  Work item: (b, hkv, KV block), blocks of
 // one (b, hkv) consecutive so that they share an XCD (and its L2) and heavy /
 // light causal blocks interleave; block 0 has the longest causal band.
-template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, int PASS, bool BLK, int TPS = 1>
+template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, int PASS, bool BLK, bool DOC, int TPS = 1>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KvCfg<D>::WPE, KvCfg<D>::WPE)))
 void bwd_kv_kernel(BwdArgs a) {
   __shared__ __attribute__((aligned(1024))) char smem[KvCfg<D, TPS>::LDSB];
@@ -977,7 +994,7 @@ void bwd_kv_kernel(BwdArgs a) {
     kb = w % nkb;
     bh = w / nkb;
   }
-  kv_tile_stream<T, D, SOFTCAP, ALIBI, DS, PASS, BLK, TPS>(a, smem, slot, kb, bh);
+  kv_tile_stream<T, D, SOFTCAP, ALIBI, DS, PASS, BLK, DOC, TPS>(a, smem, slot, kb, bh);
 }
 
 // D = 256: the dV pass (PASS 1) and the dK pass (PASS 2) of every KV block in
@@ -988,7 +1005,7 @@ void bwd_kv_kernel(BwdArgs a) {
 // (at config 4, 132 query tiles then 128 .. 4 per CU, against 99 on average).
 // Item k of a group: KV block k / 2, the dK pass for even k (the longer of the
 // two per tile: dP MFMAs and the staged dS stores) and the dV pass for odd k.
-template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, bool BLK>
+template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, bool BLK, bool DOC>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KvCfg<D>::WPE, KvCfg<D>::WPE)))
 void bwd_kv_passes_kernel(BwdArgs a) {
   static_assert(KvCfg<D>::PASSES, "two passes at D = 256 only");
@@ -1002,8 +1019,8 @@ void bwd_kv_passes_kernel(BwdArgs a) {
     k = w % nit;
     bh = w / nit;
   }
-  if ((k & 1) == 0) kv_tile_stream<T, D, SOFTCAP, ALIBI, DS, 2, BLK>(a, smem, slot, k >> 1, bh);
-  else kv_tile_stream<T, D, SOFTCAP, ALIBI, false, 1, BLK>(a, smem, slot, k >> 1, bh);
+  if ((k & 1) == 0) kv_tile_stream<T, D, SOFTCAP, ALIBI, DS, 2, BLK, DOC>(a, smem, slot, k >> 1, bh);
+  else kv_tile_stream<T, D, SOFTCAP, ALIBI, false, 1, BLK, DOC>(a, smem, slot, k >> 1, bh);
 }
 
 #ifndef FLEXATT_KV_TPS
@@ -1016,62 +1033,44 @@ hipError_t launch_kv(const BwdArgs& a, hipStream_t st) {
   static_assert(C::BKV == kDsKB && C::BM == kDsQT, "staged dS units are one tile by one KV block");
   BwdArgs x = a;
   x.ntiles = (a.p.Skv + C::BKV - 1) / C::BKV;
-  const dim3 grid(x.ntiles * a.p.B * a.p.Hkv), block(C::NW * 64);
-  const bool sc = a.p.cap > 0.f, al = a.p.alibi != nullptr;
-  auto go = [&](auto pass_c) {
-    constexpr int PS = decltype(pass_c)::value;
-    constexpr bool DSP = DS && PS != 1;
-    x.queue = a.queue;
-    // block-sparse maps: the walk list of live query tiles in dynamic LDS
-    // (when it fits beside the tile stages; otherwise removed tiles are walked
-    // and only their S-wave work is skipped)
-    const size_t dyn = 2 * (size_t)((a.p.Sq + C::BM - 1) / C::BM + 2);
-    if (a.p.blk && C::LDSB + dyn <= 160 * 1024) {
-      if (sc && al) hipLaunchKernelGGL((bwd_kv_kernel<T, D, true, true, DSP, PS, true>), grid, block, dyn, st, x);
-      else if (sc) hipLaunchKernelGGL((bwd_kv_kernel<T, D, true, false, DSP, PS, true>), grid, block, dyn, st, x);
-      else if (al) hipLaunchKernelGGL((bwd_kv_kernel<T, D, false, true, DSP, PS, true>), grid, block, dyn, st, x);
-      else hipLaunchKernelGGL((bwd_kv_kernel<T, D, false, false, DSP, PS, true>), grid, block, dyn, st, x);
-      return hipGetLastError();
-    }
-    if constexpr (D == 128 && PS == 0 && FLEXATT_KV_TPS == 2) {
-      if (!a.p.blk) {
-        constexpr int TP = FLEXATT_KV_TPS;
-        if (sc && al) hipLaunchKernelGGL((bwd_kv_kernel<T, D, true, true, DSP, PS, false, TP>), grid, block, 0, st, x);
-        else if (sc) hipLaunchKernelGGL((bwd_kv_kernel<T, D, true, false, DSP, PS, false, TP>), grid, block, 0, st, x);
-        else if (al) hipLaunchKernelGGL((bwd_kv_kernel<T, D, false, true, DSP, PS, false, TP>), grid, block, 0, st, x);
-        else hipLaunchKernelGGL((bwd_kv_kernel<T, D, false, false, DSP, PS, false, TP>), grid, block, 0, st, x);
-        return hipGetLastError();
+  const int items = x.ntiles * a.p.B * a.p.Hkv;
+  const dim3 block(C::NW * 64);
+  // block-sparse maps: the walk list of live query tiles in dynamic LDS
+  // (when it fits beside the tile stages; otherwise removed tiles are walked
+  // and only their S-wave work is skipped)
+  const size_t list = 2 * (size_t)((a.p.Sq + C::BM - 1) / C::BM + 2);
+  const bool blk = a.p.blk && C::LDSB + list <= 160 * 1024;
+  const size_t dyn = blk ? list : 0;
+  auto go = [&](auto sc, auto al, auto bl, auto doc) {
+    constexpr bool SC = decltype(sc)::value, AL = decltype(al)::value, BL = decltype(bl)::value,
+                   DOC = decltype(doc)::value;
+    if constexpr (C::PASSES) {  // both passes' items in one launch
+      hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, SC, AL, DS, BL, DOC>), dim3(2 * items), block, dyn, st, x);
+    } else {
+      if constexpr (D == 128 && !BL && FLEXATT_KV_TPS == 2) {
+        if (!a.p.blk) {
+          hipLaunchKernelGGL((bwd_kv_kernel<T, D, SC, AL, DS, 0, BL, DOC, FLEXATT_KV_TPS>), dim3(items), block, dyn, st,
+                             x);
+          return;
+        }
       }
+      hipLaunchKernelGGL((bwd_kv_kernel<T, D, SC, AL, DS, 0, BL, DOC>), dim3(items), block, dyn, st, x);
     }
-    if (sc && al) hipLaunchKernelGGL((bwd_kv_kernel<T, D, true, true, DSP, PS, false>), grid, block, 0, st, x);
-    else if (sc) hipLaunchKernelGGL((bwd_kv_kernel<T, D, true, false, DSP, PS, false>), grid, block, 0, st, x);
-    else if (al) hipLaunchKernelGGL((bwd_kv_kernel<T, D, false, true, DSP, PS, false>), grid, block, 0, st, x);
-    else hipLaunchKernelGGL((bwd_kv_kernel<T, D, false, false, DSP, PS, false>), grid, block, 0, st, x);
-    return hipGetLastError();
   };
-  if constexpr (C::PASSES) {
-    {
-      // both passes in one launch (bwd_kv_passes_kernel)
-      const dim3 grid2(2 * x.ntiles * a.p.B * a.p.Hkv);
-      x.queue = a.queue;
-      const size_t dyn = 2 * (size_t)((a.p.Sq + C::BM - 1) / C::BM + 2);
-      const bool blk = a.p.blk && C::LDSB + dyn <= 160 * 1024;
-      if (blk) {
-        if (sc && al) hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, true, true, DS, true>), grid2, block, dyn, st, x);
-        else if (sc) hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, true, false, DS, true>), grid2, block, dyn, st, x);
-        else if (al) hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, false, true, DS, true>), grid2, block, dyn, st, x);
-        else hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, false, false, DS, true>), grid2, block, dyn, st, x);
-      } else {
-        if (sc && al) hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, true, true, DS, false>), grid2, block, 0, st, x);
-        else if (sc) hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, true, false, DS, false>), grid2, block, 0, st, x);
-        else if (al) hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, false, true, DS, false>), grid2, block, 0, st, x);
-        else hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, false, false, DS, false>), grid2, block, 0, st, x);
-      }
-      return hipGetLastError();
-    }
-  } else {
-    return go(std::integral_constant<int, 0>{});
-  }
+  using std::false_type;
+  using std::true_type;
+  auto masks = [&](auto sc, auto al) {
+    if (blk && a.p.docc) go(sc, al, true_type{}, true_type{});
+    else if (blk) go(sc, al, true_type{}, false_type{});
+    else if (a.p.docc) go(sc, al, false_type{}, true_type{});
+    else go(sc, al, false_type{}, false_type{});
+  };
+  const bool sc = a.p.cap > 0.f, al = a.p.alibi != nullptr;
+  if (sc && al) masks(true_type{}, true_type{});
+  else if (sc) masks(true_type{}, false_type{});
+  else if (al) masks(false_type{}, true_type{});
+  else masks(false_type{}, false_type{});
+  return hipGetLastError();
 }
 
 #define FLEXATT_KV_LAUNCHERS(D)                                                                     \

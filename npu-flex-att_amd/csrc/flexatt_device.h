@@ -395,6 +395,17 @@ __device__ __forceinline__ void col_bounds(const Shape& p, int b, int j, int& lo
     hi = 0x7fffffff;
   }
 }
+// Interval masks in the staged backward: the query rows [lo, hi) some key of
+// KV block kb (kDsKB keys) may meet.  The bounds are non-decreasing, so the
+// block's first and last key give them, and over kb both are non-decreasing
+// too.  The dK/dV kernels walk (and store the dS of) only the query tiles
+// floor(lo / kDsQT) .. ceil(hi / kDsQT) - 1 of a block, and the dQ kernels
+// read exactly those units (ds_doc_range).
+__device__ __forceinline__ void kb_col_range(const Shape& p, int b, int kb, int& lo, int& hi) {
+  const int2* c = (const int2*)p.docc + (int64_t)b * p.Skv;
+  lo = max(c[min(kb * 128, p.Skv - 1)].x, 0);
+  hi = min(c[min(kb * 128 + 127, p.Skv - 1)].y, p.Sq);
+}
 // Block-sparse mask: whether the 128 x 128 block holding (query row i, key j)
 // of head hq is computed (true when no block map is set).
 constexpr int kBlk = 128;
@@ -456,6 +467,24 @@ __host__ __device__ __forceinline__ int64_t ds_tile_offset(int t, int causal, in
   const int64_t hi = causal ? ds_quarter_sum((int64_t)t + 4, nkb) : (int64_t)t * nkb;
   const int64_t lo = window > 0 ? ds_quarter_sum((int64_t)t - (window + kDsQT - 1) / kDsQT, nkb) : 0;
   return hi - lo;
+}
+
+// The KV blocks [lo, hi) whose walk includes query tile t under an interval
+// mask: those with ceil(hi_kb / 32) > t form a suffix and those with
+// floor(lo_kb / 32) <= t a prefix of the blocks (kb_col_range is
+// non-decreasing).  Counted with ballots, one KV block per lane; every lane of
+// the wave calls it with the same t.
+__device__ __forceinline__ void ds_doc_range(const Shape& p, int b, int t, int nkb, int& lo, int& hi) {
+  int before = 0, reach = 0;
+  for (int k0 = 0; k0 < nkb; k0 += 64) {
+    const int kb = k0 + (threadIdx.x & 63);
+    int l = 0, h = 0;
+    kb_col_range(p, b, min(kb, nkb - 1), l, h);
+    before += __builtin_popcountll(__builtin_amdgcn_ballot_w64(kb < nkb && h <= t * kDsQT));
+    reach += __builtin_popcountll(__builtin_amdgcn_ballot_w64(kb < nkb && l < (t + 1) * kDsQT));
+  }
+  lo = before;
+  hi = reach;
 }
 
 // allowed(i, j) for the masks of the path (j < Skv is the KV tail).
