@@ -99,6 +99,13 @@ typedef struct flexatt_problem {
   int32_t reserved; /* 0 */
 } flexatt_problem;
 
+/* The interval bounds of a document mask (flexatt_problem.doc_bounds) from
+ * document ids: `ids` is a contiguous device array [batch, seqlen] of integers
+ * of ids_bytes (1, 2, 4 or 8) bytes, and bounds[b][s] receives the range
+ * [lo, hi) of the maximal run of equal ids that holds position s.  No
+ * counterpart in the reference. */
+int flexatt_document_bounds(const void* ids, int ids_bytes, int batch, int seqlen, int32_t* bounds, void* stream);
+
 /* Forward: o = softmax(mask(score(q k^T))) v and lse.
  * Replaces the flash_attn_fwd_kernel launch of npu_flash_attention_forward,
  * npu_flash_attention.py:634-652. */

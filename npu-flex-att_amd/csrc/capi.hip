@@ -475,6 +475,14 @@ int flexatt_fwd_decode_noalloc(const flexatt_problem* p, const flexatt_tensor* q
   return decode_run(p, d, q, k, v, o, lse, ws, (hipStream_t)stream);
 }
 
+int flexatt_document_bounds(const void* ids, int ids_bytes, int batch, int seqlen, int32_t* bounds, void* stream) {
+  if (!ids || !bounds || batch <= 0 || seqlen <= 0) return FLEXATT_EINVAL;
+  if (ids_bytes != 1 && ids_bytes != 2 && ids_bytes != 4 && ids_bytes != 8) return FLEXATT_EINVAL;
+  if ((uintptr_t)ids % ids_bytes != 0 || (uintptr_t)bounds % sizeof(int32_t) != 0) return FLEXATT_ELAYOUT;
+  if ((int64_t)batch * seqlen > INT32_MAX) return FLEXATT_ESHAPE;
+  return (int)doc_bounds_run(ids, ids_bytes, batch, seqlen, bounds, (hipStream_t)stream);
+}
+
 namespace {
 int run_delta(const flexatt_problem* p, const flexatt_tensor* o, const flexatt_tensor* dout, float* delta,
               int* zero, void* stream) {

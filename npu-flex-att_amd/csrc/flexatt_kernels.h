@@ -81,6 +81,10 @@ hipError_t fwd_ws_bf16_d256(const FwdArgs&, hipStream_t);
 hipError_t fwd_ws_f16_d256(const FwdArgs&, hipStream_t);
 bool fwd_ws_fits(const Shape& p);  // its LDS (with a block map's lists) fits one CU
 
+// [lo, hi) of every position's document (doc_bounds.hip): ids [B][S] integers
+// of ids_bytes bytes, bounds int32 [B][S][2].
+hipError_t doc_bounds_run(const void* ids, int ids_bytes, int B, int S, int* bounds, hipStream_t);
+
 hipError_t bwd_delta(int dtype, const DeltaArgs&, hipStream_t);
 
 // Split-KV decode forward (fwd_decode.hip), D <= 128.

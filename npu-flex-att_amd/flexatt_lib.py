@@ -16,6 +16,7 @@ F32, F16, BF16 = 0, 1, 2
 
 # Entry points declared in include/flexatt.h.
 EXPORTS = (
+    "flexatt_document_bounds",
     "flexatt_fwd",
     "flexatt_fwd_decode_workspace",
     "flexatt_fwd_decode",
@@ -99,6 +100,7 @@ def load() -> ctypes.CDLL:
     fp = ctypes.c_void_p
     st = ctypes.c_void_p
     sig = {
+        "flexatt_document_bounds": [fp, ctypes.c_int, ctypes.c_int, ctypes.c_int, fp, st],
         "flexatt_fwd": [pr, T, T, T, T, fp, st],
         "flexatt_fwd_decode": [pr, T, T, T, T, fp, fp, ctypes.c_size_t, st],
         "flexatt_fwd_decode_noalloc": [pr, T, T, T, T, fp, st],

@@ -159,11 +159,12 @@ def _alibi(alibi_slope, hq, device):
     return s
 
 
-def _doc_bounds(document_ids, B, Sq, Sk, device):
+def _doc_bounds(document_ids, B, Sq, Sk, device, native=False):
     """Document masks: ``document_ids`` [B, S] (S = Sq = Skv) -> int32
     [B, S, 2] holding, per position, the range [lo, hi) of its document, a
     maximal run of equal ids.  Positions of different documents do not attend
-    to each other."""
+    to each other.  ``native``: one kernel of the library (device tensors of
+    an eager call) instead of tensor operations (which can be traced)."""
     if document_ids is None:
         return None
     ids = torch.as_tensor(document_ids, device=device)
@@ -172,6 +173,14 @@ def _doc_bounds(document_ids, B, Sq, Sk, device):
     if ids.dtype.is_floating_point or ids.dtype == torch.bool:
         raise RuntimeError("document_ids must be an integer tensor")
     S = Sk
+    if native and ids.is_cuda and ids.numel() > 0:
+        ids = ids.contiguous()
+        bounds = torch.empty(B, S, 2, dtype=torch.int32, device=ids.device)
+        with torch.cuda.device(ids.device):
+            st = _lib.load().flexatt_document_bounds(ids.data_ptr(), ids.element_size(), B, S, bounds.data_ptr(),
+                                                     _stream(ids.device))
+        _lib.check(st, "flexatt_document_bounds")
+        return bounds
     pos = torch.arange(S, device=device, dtype=torch.int32).expand(B, S)
     start = torch.ones(B, S, dtype=torch.bool, device=device)
     start[:, 1:] = ids[:, 1:] != ids[:, :-1]
@@ -275,11 +284,12 @@ def _block_map(block_mask, B, Hq, Sq, Sk, device):
     return m.to(device=device, dtype=torch.uint8).expand(B, m.shape[1], nq, nk).contiguous()
 
 
-def _masks(causal, document_ids, prefix_len, block_mask, B, Hq, Sq, Sk, device):
-    """The interval / block masks of one call as kernel inputs, or None."""
+def _masks(causal, document_ids, prefix_len, block_mask, B, Hq, Sq, Sk, device, native=False):
+    """The interval / block masks of one call as kernel inputs, or None
+    (``native``: see :func:`_doc_bounds`)."""
     if document_ids is None and block_mask is None and (prefix_len is None or not causal):
         return None
-    rows = _doc_bounds(document_ids, B, Sq, Sk, device)
+    rows = _doc_bounds(document_ids, B, Sq, Sk, device, native)
     cols = None
     if prefix_len is not None and causal:
         rows, cols = _prefix_bounds(prefix_len, rows, B, Sq, Sk, device)
@@ -333,7 +343,7 @@ def npu_flash_attention_forward(
     if not _kernel_ready(O):
         O = torch.empty(query.shape, dtype=query.dtype, device=query.device)
     LSE = torch.empty(B, Hq, Sq, device=query.device, dtype=torch.float32)
-    masks = _masks(causal, document_ids, prefix_len, block_mask, B, Hq, Sq, Sk, query.device)
+    masks = _masks(causal, document_ids, prefix_len, block_mask, B, Hq, Sq, Sk, query.device, native=True)
     _forward_into(query, key, value, O, LSE, causal=causal, sliding_window=sliding_window,
                   alibi=alibi_slope, scale=scale, soft_cap=soft_cap, masks=masks)
     if return_lse:
@@ -409,7 +419,7 @@ def npu_flash_attention_backward(
         DQ = torch.empty(query.shape, dtype=query.dtype, device=query.device)
     DK = torch.empty(B, Hkv, Sk, D, device=key.device, dtype=key.dtype)
     DV = torch.empty(B, Hkv, Sk, D, device=value.device, dtype=value.dtype)
-    masks = _masks(causal, document_ids, prefix_len, block_mask, B, Hq, Sq, Sk, query.device)
+    masks = _masks(causal, document_ids, prefix_len, block_mask, B, Hq, Sq, Sk, query.device, native=True)
     _backward_into(query, key, value, out, lse, grad_out, DQ, DK, DV, causal=causal,
                    sliding_window=sliding_window, alibi=alibi_slope, scale=scale, soft_cap=soft_cap, masks=masks)
     return DQ, DK, DV
