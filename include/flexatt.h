@@ -128,6 +128,14 @@ int flexatt_fwd_decode(const flexatt_problem* p, const flexatt_tensor* q, const 
                        const flexatt_tensor* v, const flexatt_tensor* o, float* lse, void* workspace,
                        size_t workspace_bytes, void* stream);
 
+/* The split-KV forward over its whole range: that of flexatt_fwd_decode and
+ * head_dim 256 (else FLEXATT_ERANGE, and 0 bytes); otherwise as
+ * flexatt_fwd_decode. */
+size_t flexatt_fwd_split_workspace(const flexatt_problem* p); /* 0: outside the range */
+int flexatt_fwd_split(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
+                      const flexatt_tensor* v, const flexatt_tensor* o, float* lse, void* workspace,
+                      size_t workspace_bytes, void* stream);
+
 /* Split-KV decode forward that allocates nothing.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory or pass a
  * workspace (code under HIP graph capture, tight serving loops, harnesses

@@ -147,11 +147,14 @@ const BwdLauncher kDkdv[3][4] = {
 // Split-KV decode: range, plan and workspace.
 constexpr int kDecWaves = 4;  // waves per workgroup
 constexpr int kDecTile = 32;   // KV rows per tile
-bool decode_applies(const flexatt_problem* p) {
-  return (p->dtype == FLEXATT_F16 || p->dtype == FLEXATT_BF16) && p->head_dim <= 128 && !p->doc_bounds &&
-         !p->block_map &&
+bool is_16bit(const flexatt_problem* p) { return p->dtype == FLEXATT_F16 || p->dtype == FLEXATT_BF16; }
+// flexatt_fwd_split: the query rows of a KV head fit one 32-row tile.
+bool split_applies(const flexatt_problem* p) {
+  return is_16bit(p) && !p->doc_bounds && !p->block_map &&
          (int64_t)(p->heads_q / p->heads_kv) * p->seqlen_q <= 32;
 }
+// flexatt_fwd_decode (and _noalloc): the same at head_dim <= 128.
+bool decode_applies(const flexatt_problem* p) { return split_applies(p) && p->head_dim <= 128; }
 struct DecodePlan {
   int nsplit, chunk, ntiles;
   size_t bytes;  // workspace: partial O then partial LSE
@@ -175,16 +178,17 @@ DecodePlan decode_plan(const flexatt_problem* p) {
   d.bytes = (size_t)(rows * parts * (p->head_dim + 1) * (int64_t)sizeof(float));
   return d;
 }
-const DecodeLauncher kDecode[3][3] = {
-    {nullptr, nullptr, nullptr},
-    {fwd_decode_f16_d32, fwd_decode_f16_d64, fwd_decode_f16_d128},
-    {fwd_decode_bf16_d32, fwd_decode_bf16_d64, fwd_decode_bf16_d128},
+const DecodeLauncher kSplit[3][4] = {
+    {nullptr, nullptr, nullptr, nullptr},
+    {fwd_split_f16_d32, fwd_split_f16_d64, fwd_split_f16_d128, fwd_split_f16_d256},
+    {fwd_split_bf16_d32, fwd_split_bf16_d64, fwd_split_bf16_d128, fwd_split_bf16_d256},
 };
 
 // Launch the decode kernels with their partials in `ws` (d.bytes, 16-byte
 // aligned); the problem and tensors are already checked.
 int decode_run(const flexatt_problem* p, const DecodePlan& d, const flexatt_tensor* q, const flexatt_tensor* k,
-               const flexatt_tensor* v, const flexatt_tensor* o, float* lse, void* ws, hipStream_t stream) {
+               const flexatt_tensor* v, const flexatt_tensor* o, float* lse, void* ws, hipStream_t stream,
+               int nw = kDecWaves) {
   DecodeArgs a;
   a.q = view(q);
   a.k = view(k);
@@ -194,11 +198,12 @@ int decode_run(const flexatt_problem* p, const DecodePlan& d, const flexatt_tens
   a.p = make_shape(p);
   a.nsplit = d.nsplit;
   a.chunk = d.chunk;
-  a.ntiles = d.ntiles;
+  a.nw = nw;
+  a.nrt = 0;
   const int64_t rows = (int64_t)p->batch * p->heads_q * p->seqlen_q;
   a.part_o = (float*)ws;
   a.part_lse = a.part_o + rows * d.nsplit * p->head_dim;
-  return (int)kDecode[p->dtype][head_index(p->head_dim)](a, stream);
+  return (int)kSplit[p->dtype][head_index(p->head_dim)](a, stream);
 }
 
 // Fixed partial-result buffer of flexatt_fwd_decode_noalloc: one copy per GPU,
@@ -275,6 +280,55 @@ int cu_count() {
     cache[dev].store(n, std::memory_order_relaxed);
   }
   return n;
+}
+
+// Attended (query row, key) pairs of one head under the causal and window
+// masks (interval masks, whose bounds are on the device, not counted).
+int64_t attended_pairs(const flexatt_problem* p) {
+  const int64_t n = p->seqlen_q, m = p->seqlen_kv, w = p->sliding_window;
+  auto tri = [](int64_t x) { return x > 0 ? x * (x + 1) / 2 : 0; };
+  // sum over rows i of the row's end (i + 1 capped at m, or m) ...
+  int64_t sum = !p->causal ? n * m : n <= m ? tri(n) : tri(m) + (n - m) * m;
+  if (w > 0) {
+    // ... less its start i - w, and less the whole row once the start reaches m
+    const int64_t live = n < m + w ? n : m + w;  // rows that keep a key
+    sum -= tri(live - 1 - w) + (n - live) * m;
+  }
+  return sum;
+}
+
+// Waves per workgroup of the forward that splits a 32-row tile's keys over
+// the waves (fwd_split.hip, one workgroup per row tile), or 0 for the regular
+// forward.  The regular workgroup covers 256 query rows and walks their keys as
+// one chain, so its time is the longest chain until its grid fills the chip;
+// the split workgroup covers 32 rows, shortens the chain by its wave count and
+// costs about twice the regular kernel's time per pair.  Measured at the
+// crossover, in tiles of 32 x 32 pairs per CU (U / CUs) against the longest
+// chain L in 32-key tiles (bf16, regular -> split, us): D = 128: U = 2 CUs L
+// B=1 Hq=32 Hkv=8 S=1024 causal 27.0 -> 23.4, non-causal (4 CUs L) 26.9 -> 34.1;
+// D = 64: 4 CUs L, the same heads at S=2048 causal 39.8 -> 34.6, non-causal
+// (8 CUs L) 42.8 -> 61.5; D = 256: one workgroup per CU, Hq=16 S=512 19.4 ->
+// 15.6, S=1024 30.7 -> 31.3.  Far from it: B=1 H=2 D=64 S=2048 39.4 -> 10.7, S=128
+// 6.7 -> 4.4.
+// Eight waves instead of four where the chip has a CU per workgroup and the
+// chain is long enough to pay for the larger combine: H=2 D=64 S=2048 14.0 ->
+// 10.7, Hq=8 Hkv=2 D=128 S=2048 causal 27.2 -> 23.1 but non-causal 31.0 -> 34.4,
+// S=512 8.1 -> 8.9.
+int split_waves(const flexatt_problem* p) {
+  if (!is_16bit(p) || p->block_map) return 0;
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  const int64_t G = p->heads_q / p->heads_kv, groups = (int64_t)p->batch * p->heads_kv;
+  const int64_t wgs = groups * ((G * p->seqlen_q + 31) / 32);
+  int64_t keys = p->causal && p->seqlen_q < p->seqlen_kv ? p->seqlen_q : p->seqlen_kv;  // the longest row's
+  if (p->sliding_window > 0) {
+    const int64_t w = (int64_t)p->sliding_window + (p->causal ? 32 : p->seqlen_kv);
+    if (w < keys) keys = w;
+  }
+  const int64_t chain = (keys + 31) / 32;
+  const int64_t units = groups * G * attended_pairs(p) / (32 * 32) + wgs / 2;  // and the tiles' masked edges
+  if (p->head_dim == 256) return wgs <= cus ? 4 : 0;
+  if (units > (p->head_dim == 128 ? 2 : 4) * cus * chain) return 0;
+  return wgs <= cus && chain >= (p->head_dim == 128 ? 64 : 32) && (p->head_dim < 128 || 2 * units <= cus * chain) ? 8 : 4;
 }
 
 int bwd_common(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
@@ -424,6 +478,11 @@ int flexatt_fwd(const flexatt_problem* p, const flexatt_tensor* q, const flexatt
   FLEXATT_TRY(check_tensor(v, p->dtype));
   FLEXATT_TRY(check_out_tensor(o, p->dtype, p->batch, p->heads_q, p->seqlen_q, p->head_dim));
   if (!lse) return FLEXATT_EINVAL;
+  const int nw = split_waves(p);
+  if (nw) {
+    const DecodePlan d{1, 0, 0, 0};
+    return decode_run(p, d, q, k, v, o, lse, nullptr, (hipStream_t)stream, nw);
+  }
   FwdArgs a;
   a.q = view(q);
   a.k = view(k);
@@ -450,6 +509,28 @@ int flexatt_fwd_decode(const flexatt_problem* p, const flexatt_tensor* q, const 
   FLEXATT_TRY(check_out_tensor(o, p->dtype, p->batch, p->heads_q, p->seqlen_q, p->head_dim));
   if (!lse || !workspace) return FLEXATT_EINVAL;
   if (!decode_applies(p)) return FLEXATT_ERANGE;
+  const DecodePlan d = decode_plan(p);
+  if (workspace_bytes < d.bytes) return FLEXATT_EINVAL;
+  if (((uintptr_t)workspace) % 16 != 0) return FLEXATT_ELAYOUT;
+  if (d.ntiles == 0) return FLEXATT_EINVAL;
+  return decode_run(p, d, q, k, v, o, lse, workspace, (hipStream_t)stream);
+}
+
+size_t flexatt_fwd_split_workspace(const flexatt_problem* p) {
+  if (check_problem(p) != FLEXATT_OK || !split_applies(p)) return 0;
+  return decode_plan(p).bytes;
+}
+
+int flexatt_fwd_split(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
+                      const flexatt_tensor* v, const flexatt_tensor* o, float* lse, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+  FLEXATT_TRY(check_problem(p));
+  FLEXATT_TRY(check_tensor(q, p->dtype));
+  FLEXATT_TRY(check_tensor(k, p->dtype));
+  FLEXATT_TRY(check_tensor(v, p->dtype));
+  FLEXATT_TRY(check_out_tensor(o, p->dtype, p->batch, p->heads_q, p->seqlen_q, p->head_dim));
+  if (!lse || !workspace) return FLEXATT_EINVAL;
+  if (!split_applies(p)) return FLEXATT_ERANGE;
   const DecodePlan d = decode_plan(p);
   if (workspace_bytes < d.bytes) return FLEXATT_EINVAL;
   if (((uintptr_t)workspace) % 16 != 0) return FLEXATT_ELAYOUT;

@@ -45,7 +45,8 @@ struct BwdArgs {
   int nstatic;
 };
 
-// Split-KV decode forward (fwd_decode.hip): partials in the caller's workspace.
+// Split-KV forward (fwd_split.hip): partials in the caller's workspace, none
+// with one split per row tile.
 struct DecodeArgs {
   View q, k, v;
   MutView o;
@@ -53,9 +54,10 @@ struct DecodeArgs {
   float* part_o;    // [B * Hq * Sq][nsplit][D], O of each partial / its row sums
   float* part_lse;  // [B * Hq * Sq][nsplit], LSE of each partial in log2 units
   Shape p;
-  int nsplit;  // workgroups per (b, hkv)
-  int chunk;   // 32-row KV tiles per workgroup
-  int ntiles;  // 32-row KV tiles in the attended range
+  int nsplit;  // workgroups per row tile
+  int chunk;   // 32-row KV tiles per workgroup (nsplit > 1)
+  int nw;      // waves per workgroup with one split (4 or 8; D = 256: 4)
+  int nrt;     // 32-row tiles of packed query rows per (b, hkv) (set by the launcher)
 };
 
 typedef hipError_t (*FwdLauncher)(const FwdArgs&, hipStream_t);
@@ -87,13 +89,15 @@ hipError_t doc_bounds_run(const void* ids, int ids_bytes, int B, int S, int* bou
 
 hipError_t bwd_delta(int dtype, const DeltaArgs&, hipStream_t);
 
-// Split-KV decode forward (fwd_decode.hip), D <= 128.
-hipError_t fwd_decode_bf16_d32(const DecodeArgs&, hipStream_t);
-hipError_t fwd_decode_f16_d32(const DecodeArgs&, hipStream_t);
-hipError_t fwd_decode_bf16_d64(const DecodeArgs&, hipStream_t);
-hipError_t fwd_decode_f16_d64(const DecodeArgs&, hipStream_t);
-hipError_t fwd_decode_bf16_d128(const DecodeArgs&, hipStream_t);
-hipError_t fwd_decode_f16_d128(const DecodeArgs&, hipStream_t);
+// Split-KV forward (fwd_split.hip).
+hipError_t fwd_split_bf16_d32(const DecodeArgs&, hipStream_t);
+hipError_t fwd_split_f16_d32(const DecodeArgs&, hipStream_t);
+hipError_t fwd_split_bf16_d64(const DecodeArgs&, hipStream_t);
+hipError_t fwd_split_f16_d64(const DecodeArgs&, hipStream_t);
+hipError_t fwd_split_bf16_d128(const DecodeArgs&, hipStream_t);
+hipError_t fwd_split_f16_d128(const DecodeArgs&, hipStream_t);
+hipError_t fwd_split_bf16_d256(const DecodeArgs&, hipStream_t);
+hipError_t fwd_split_f16_d256(const DecodeArgs&, hipStream_t);
 
 // dK/dV as a KV-stationary tile stream (bwd_kv.hip), D = 64, 128 and 256.
 hipError_t bwd_kv_bf16_d128(const BwdArgs&, hipStream_t);

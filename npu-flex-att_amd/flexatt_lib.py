@@ -20,6 +20,8 @@ EXPORTS = (
     "flexatt_fwd",
     "flexatt_fwd_decode_workspace",
     "flexatt_fwd_decode",
+    "flexatt_fwd_split_workspace",
+    "flexatt_fwd_split",
     "flexatt_fwd_decode_noalloc",
     "flexatt_bwd_delta",
     "flexatt_bwd_dq",
@@ -103,6 +105,7 @@ def load() -> ctypes.CDLL:
         "flexatt_document_bounds": [fp, ctypes.c_int, ctypes.c_int, ctypes.c_int, fp, st],
         "flexatt_fwd": [pr, T, T, T, T, fp, st],
         "flexatt_fwd_decode": [pr, T, T, T, T, fp, fp, ctypes.c_size_t, st],
+        "flexatt_fwd_split": [pr, T, T, T, T, fp, fp, ctypes.c_size_t, st],
         "flexatt_fwd_decode_noalloc": [pr, T, T, T, T, fp, st],
         "flexatt_bwd_delta": [pr, T, T, fp, st],
         "flexatt_bwd_dq": [pr, T, T, T, T, fp, fp, T, st],
@@ -117,7 +120,7 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.argtypes = args
         fn.restype = ctypes.c_int
-    for name in ("flexatt_fwd_decode_workspace", "flexatt_bwd_workspace"):
+    for name in ("flexatt_fwd_decode_workspace", "flexatt_fwd_split_workspace", "flexatt_bwd_workspace"):
         getattr(lib, name).argtypes = [pr]
         getattr(lib, name).restype = ctypes.c_size_t
     lib.flexatt_bwd_workspace_limited.argtypes = [pr, ctypes.c_size_t]

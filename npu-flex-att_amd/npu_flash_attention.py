@@ -54,8 +54,8 @@ __all__ = [
 
 _DTYPES = {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 
-# The forward takes the split-KV decode kernels (flexatt_fwd_decode) whenever
-# the problem is in their range: fp16/bf16, D <= 128 and (Hq / Hkv) * Sq <= 32.
+# The forward splits the KV range over workgroups (flexatt_fwd_split) whenever
+# the problem is in that range: fp16/bf16 and (Hq / Hkv) * Sq <= 32 (decoding).
 # Set to False to force the regular forward kernel (tests compare the two).
 decode_enabled = True
 # The backward stages dS through a workspace (flexatt_bwd_ws) whenever the
@@ -364,13 +364,13 @@ def _forward_into(query, key, value, O, LSE, *, causal, sliding_window, alibi, s
     p = _problem(q, k, scale, causal, sliding_window, soft_cap, slopes, masks)
     # Few query rows per KV head (decoding): the split-KV kernels, with their
     # partial results in a workspace from torch's caching allocator.
-    ws_bytes = lib.flexatt_fwd_decode_workspace(p) if decode_enabled else 0
+    ws_bytes = lib.flexatt_fwd_split_workspace(p) if decode_enabled else 0
     with torch.cuda.device(query.device):
         if ws_bytes:
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device)
-            st = lib.flexatt_fwd_decode(p, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v), _lib.tensor(O),
-                                        LSE.data_ptr(), ws.data_ptr(), ws_bytes, _stream(query.device))
-            _lib.check(st, "flexatt_fwd_decode")
+            st = lib.flexatt_fwd_split(p, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v), _lib.tensor(O),
+                                       LSE.data_ptr(), ws.data_ptr(), ws_bytes, _stream(query.device))
+            _lib.check(st, "flexatt_fwd_split")
             return
         st = lib.flexatt_fwd(p, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v), _lib.tensor(O),
                              LSE.data_ptr(), _stream(query.device))
