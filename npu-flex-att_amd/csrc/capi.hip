@@ -325,10 +325,13 @@ int split_waves(const flexatt_problem* p) {
     if (w < keys) keys = w;
   }
   const int64_t chain = (keys + 31) / 32;
-  const int64_t units = groups * G * attended_pairs(p) / (32 * 32) + wgs / 2;  // and the tiles' masked edges
+  const int64_t units = groups * G * attended_pairs(p) / (32 * 32);
   if (p->head_dim == 256) return wgs <= cus ? 4 : 0;
-  if (units > (p->head_dim == 128 ? 2 : 4) * cus * chain) return 0;
-  return wgs <= cus && chain >= (p->head_dim == 128 ? 64 : 32) && (p->head_dim < 128 || 2 * units <= cus * chain) ? 8 : 4;
+  // (an eighth above the measured points, whose causal pairs are just over half)
+  const int64_t load = 8 * units / (cus * chain);  // in eighths
+  if (load > (p->head_dim == 128 ? 18 : 36)) return 0;
+  if (p->head_dim == 128) return wgs <= cus && chain >= 64 && load <= 9 ? 8 : 4;
+  return wgs <= cus && chain >= 32 ? 8 : 4;
 }
 
 int bwd_common(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,

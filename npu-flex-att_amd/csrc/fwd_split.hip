@@ -171,7 +171,13 @@ void fwd_split_kernel(DecodeArgs a) {
     }
     if (c2 == 0.f) c2 = 1e-30f;
   }
-  const float slope_log2 = ALIBI ? p.alibi[hq] * kLog2e : 0.f;
+  float slope_log2 = ALIBI ? p.alibi[hq] * kLog2e : 0.f;
+  // Wait for Q here, once, together with the first tile: without the pins the
+  // compiler waits at the first use, inside the tile loop, where its vmcnt(0)
+  // drains the copies in flight on every tile.
+#pragma unroll
+  for (int kc = 0; kc < C::KC; ++kc) pin(qf[kc]);
+  if constexpr (ALIBI) pin(slope_log2);
 
   int koff[C::KC], voff[C::DB];
   {
