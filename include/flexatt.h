@@ -250,6 +250,23 @@ int flexatt_bwd_ws(const flexatt_problem* p, const flexatt_tensor* q, const flex
                    const float* lse, float* delta, const flexatt_tensor* dq, const flexatt_tensor* dk,
                    const flexatt_tensor* dv, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Whole backward for problems that fill few workgroups of the other two: the
+ * Delta pass into `delta`, then dK/dV and dQ in one launch whose items split
+ * their streams of tiles over the waves of a workgroup, and the long dK/dV
+ * streams over several workgroups (fp32 sums in the workspace, added by one
+ * more launch).  Range: fp16/bf16 at head_dim <= 128 without a block map (else
+ * FLEXATT_ERANGE).  `workspace`: flexatt_bwd_split_workspace(p) bytes, 16-byte
+ * aligned, not zeroed, reusable once the call's work on `stream` is done; NULL
+ * when that is 0.  Same results as flexatt_bwd up to fp32 summation order;
+ * bitwise deterministic.  flexatt_bwd_prefers_split(p): 1 where it measured
+ * faster on MI355X than the staged and the recomputing backward, else 0. */
+int flexatt_bwd_prefers_split(const flexatt_problem* p);
+size_t flexatt_bwd_split_workspace(const flexatt_problem* p);
+int flexatt_bwd_split(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
+                      const flexatt_tensor* v, const flexatt_tensor* o, const flexatt_tensor* dout,
+                      const float* lse, float* delta, const flexatt_tensor* dq, const flexatt_tensor* dk,
+                      const flexatt_tensor* dv, void* workspace, size_t workspace_bytes, void* stream);
+
 /* The two kernels of flexatt_bwd_ws on their own (FLEXATT_ERANGE outside
  * its range).  flexatt_bwd_dkdv_ds replaces the flash_attn_bwd_dkdv_kernel
  * launch and the group sum (npu_flash_attention.py:714-737) and also fills

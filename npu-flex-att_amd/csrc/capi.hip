@@ -196,6 +196,7 @@ int decode_run(const flexatt_problem* p, const DecodePlan& d, const flexatt_tens
   a.o = mview(o);
   a.lse = lse;
   a.p = make_shape(p);
+  if (a.p.window > a.p.Sq) a.p.window = a.p.Sq;  // the same mask
   a.nsplit = d.nsplit;
   a.chunk = d.chunk;
   a.nw = nw;
@@ -647,6 +648,119 @@ int flexatt_bwd(const flexatt_problem* p, const flexatt_tensor* q, const flexatt
   a.dk = mview(dk);
   a.dv = mview(dv);
   return (int)pick_dkdv(p)(a, (hipStream_t)stream);
+}
+
+namespace {
+const BwdSplitLauncher kBwdSplit[3][4] = {
+    {nullptr, nullptr, nullptr, nullptr},
+    {bwd_split_f16_d32, bwd_split_f16_d64, bwd_split_f16_d128, nullptr},
+    {bwd_split_bf16_d32, bwd_split_bf16_d64, bwd_split_bf16_d128, nullptr},
+};
+bool bwd_split_applies(const flexatt_problem* p) {
+  return kBwdSplit[p->dtype][head_index(p->head_dim)] && !p->block_map;
+}
+// The split backward's plan, and whether it beats the staged / recomputing
+// backward, from estimates in us fitted to graph replays of 56 bf16 shapes
+// (H = 2 .. 32, G = 1 and 4, S = 128 .. 2048, B = 1 .. 4, causal, windowed and not).
+// A workgroup's time is its longest chain of 32 x 32 tiles (D = 128: 1.6 us a tile
+// and wave; 64: 1.2, 1.4 with eight waves, two to a SIMD; 32: 0.8) until the chip is full;
+// then the chip's time is `unit` per 1024 tile pairs and `wg` per 1024
+// workgroups.  The other backward's time, until its own grid fills the chip, is
+// its longest dK/dV chain (G heads of the query tiles) and its longest dQ chain.
+// Measured, other -> split (waves x splits): D = 64 H=2 S=2048 causal 75 -> 20
+// (8 x 1), Hq=8 Hkv=2 S=2048 193 -> 41 (8 x 2); D = 128 Hq=8 Hkv=2 S=1000 155
+// -> 34 (4 x 4), S=2048 286 -> 74 (4 x 2), Hq=32 Hkv=8 S=2048 295 -> 242 (4 x 1); past
+// the crossover: Hq=32 Hkv=8 B=2 S=2048 D=128 326 -> 472, D=64 242 -> 217 (not taken).
+struct BwdSplitPlan {
+  bool faster;
+  int nsplit, nw;
+  size_t bytes;
+};
+struct BwdSplitCost {
+  double tile4, tile8, base4, base8, unit, wg4, wg8, other, other_kv, other_q;
+};
+constexpr BwdSplitCost kBwdSplitCost[3] = {
+    {0.8, 1.0, 6.0, 7.0, 1.0, 5.0, 10.0, 16.0, 0.65, 0.6},   // D = 32
+    {1.2, 1.4, 7.0, 8.5, 1.4, 8.0, 14.0, 14.0, 0.62, 0.4},   // 64
+    {1.6, 0.0, 9.0, 0.0, 2.8, 20.0, 0.0, 20.0, 0.95, 0.9},   // 128 (four waves only)
+};
+BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
+  const BwdSplitCost& c = kBwdSplitCost[head_index(p->head_dim)];
+  const double G = p->heads_q / p->heads_kv, groups = (double)p->batch * p->heads_kv;
+  const int64_t nqt = (p->seqlen_q + 31) / 32, nkt = (p->seqlen_kv + 31) / 32;
+  int64_t lq = nqt, lk = nkt;  // longest streams: query tiles of a KV item, key tiles of a Q item
+  if (p->causal && nqt < lk) lk = nqt;
+  if (p->sliding_window > 0 && p->causal) {
+    const int64_t l = p->sliding_window / 32 + 2;
+    if (l < lq) lq = l;
+    if (l < lk) lk = l;
+  }
+  const double units = groups * G * (double)attended_pairs(p) / (32.0 * 32 * 1024);
+  const int64_t nrt = ((int64_t)(p->heads_q / p->heads_kv) * p->seqlen_q + 31) / 32;
+  const double part = 2.0 * sizeof(float) * groups * p->seqlen_kv * p->head_dim;  // bytes of one split's sums
+  double best = 1e30;
+  BwdSplitPlan r{false, 1, 4, 0};
+  for (int nw = 4; nw <= (p->head_dim < 128 ? 8 : 4); nw += 4)
+    for (int ns = 1; ns <= 8; ns *= 2) {
+      const double t = nw == 8 ? c.tile8 : c.tile4, base = nw == 8 ? c.base8 : c.base4;
+      const double wgs = groups * (double)(nkt * ns + nrt) / 1024;
+      const double chain = t * (G * lq / ns > lk ? G * lq / ns : lk) / nw;
+      const double work = c.unit * units + (nw == 8 ? c.wg8 : c.wg4) * wgs;
+      // the sums written and read back at about 8 TB/s (they stay in cache), and one more launch
+      const double est = base + (chain > work ? chain : work) + (ns > 1 ? 4 + 2 * ns * part / 8e6 : 0);
+      if (est < best) {
+        best = est;
+        r.nsplit = ns;
+        r.nw = nw;
+      }
+    }
+  r.faster = best < c.other + c.other_kv * G * lq + c.other_q * lk;
+  if (r.nsplit > 1) r.bytes = (size_t)(part * r.nsplit);
+  return r;
+}
+}  // namespace
+
+int flexatt_bwd_prefers_split(const flexatt_problem* p) {
+  return check_problem(p) == FLEXATT_OK && bwd_split_applies(p) && bwd_split_plan(p).faster;
+}
+
+size_t flexatt_bwd_split_workspace(const flexatt_problem* p) {
+  return check_problem(p) == FLEXATT_OK && bwd_split_applies(p) ? bwd_split_plan(p).bytes : 0;
+}
+
+int flexatt_bwd_split(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
+                      const flexatt_tensor* v, const flexatt_tensor* o, const flexatt_tensor* dout, const float* lse,
+                      float* delta, const flexatt_tensor* dq, const flexatt_tensor* dk, const flexatt_tensor* dv,
+                      void* workspace, size_t workspace_bytes, void* stream) {
+  BwdArgs c;
+  FLEXATT_TRY(bwd_common(p, q, k, v, dout, lse, delta, c));
+  FLEXATT_TRY(check_tensor(o, p->dtype));
+  FLEXATT_TRY(check_out_tensor(dq, p->dtype, p->batch, p->heads_q, p->seqlen_q, p->head_dim));
+  FLEXATT_TRY(check_out_tensor(dk, p->dtype, p->batch, p->heads_kv, p->seqlen_kv, p->head_dim));
+  FLEXATT_TRY(check_out_tensor(dv, p->dtype, p->batch, p->heads_kv, p->seqlen_kv, p->head_dim));
+  if (!bwd_split_applies(p)) return FLEXATT_ERANGE;
+  const BwdSplitPlan plan = bwd_split_plan(p);
+  if (plan.bytes && !workspace) return FLEXATT_EINVAL;
+  if (workspace_bytes < plan.bytes) return FLEXATT_EINVAL;
+  if (((uintptr_t)workspace) % 16 != 0) return FLEXATT_ELAYOUT;
+  FLEXATT_TRY(flexatt_bwd_delta(p, o, dout, delta, stream));
+  BwdSplitArgs a;
+  a.q = c.q;
+  a.k = c.k;
+  a.v = c.v;
+  a.dout = c.dout;
+  a.lse = lse;
+  a.delta = delta;
+  a.dq = mview(dq);
+  a.dk = mview(dk);
+  a.dv = mview(dv);
+  a.p = c.p;
+  if (a.p.window > a.p.Sq) a.p.window = a.p.Sq;  // the same mask, and no overflow in row + window
+  a.part = (float*)workspace;
+  a.nsplit = plan.nsplit;
+  a.nw = plan.nw;
+  a.nkt = a.nrt = 0;
+  return (int)kBwdSplit[p->dtype][head_index(p->head_dim)](a, (hipStream_t)stream);
 }
 
 size_t flexatt_bwd_workspace(const flexatt_problem* p) {

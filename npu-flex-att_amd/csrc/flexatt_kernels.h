@@ -60,9 +60,24 @@ struct DecodeArgs {
   int nrt;     // 32-row tiles of packed query rows per (b, hkv) (set by the launcher)
 };
 
+// Backward in one launch with the streams split over waves (bwd_split.hip).
+struct BwdSplitArgs {
+  View q, k, v, dout;
+  const float* lse;
+  const float* delta;
+  MutView dq, dk, dv;
+  Shape p;
+  float* part;  // nsplit > 1: [split][dK, dV][B * Hkv * Skv][D] fp32
+  int nsplit;   // workgroups per KV item
+  int nw;       // waves per workgroup (4 or 8; D = 128: 4)
+  int nkt;      // 32-row KV tiles (set by the launcher)
+  int nrt;      // 32-row tiles of packed query rows per (b, hkv) (set by the launcher)
+};
+
 typedef hipError_t (*FwdLauncher)(const FwdArgs&, hipStream_t);
 typedef hipError_t (*DecodeLauncher)(const DecodeArgs&, hipStream_t);
 typedef hipError_t (*BwdLauncher)(const BwdArgs&, hipStream_t);
+typedef hipError_t (*BwdSplitLauncher)(const BwdSplitArgs&, hipStream_t);
 
 #define FLEXATT_DECL_D(D)                                                     \
   hipError_t fwd_mfma_bf16_d##D(const FwdArgs&, hipStream_t);                 \
@@ -98,6 +113,14 @@ hipError_t fwd_split_bf16_d128(const DecodeArgs&, hipStream_t);
 hipError_t fwd_split_f16_d128(const DecodeArgs&, hipStream_t);
 hipError_t fwd_split_bf16_d256(const DecodeArgs&, hipStream_t);
 hipError_t fwd_split_f16_d256(const DecodeArgs&, hipStream_t);
+
+// Backward in one launch (bwd_split.hip), D <= 128.
+hipError_t bwd_split_bf16_d32(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_f16_d32(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_bf16_d64(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_f16_d64(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_bf16_d128(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_f16_d128(const BwdSplitArgs&, hipStream_t);
 
 // dK/dV as a KV-stationary tile stream (bwd_kv.hip), D = 64, 128 and 256.
 hipError_t bwd_kv_bf16_d128(const BwdArgs&, hipStream_t);

@@ -32,6 +32,9 @@ EXPORTS = (
     "flexatt_bwd_workspace_limited",
     "flexatt_bwd_prefers_staging",
     "flexatt_bwd_ws",
+    "flexatt_bwd_prefers_split",
+    "flexatt_bwd_split_workspace",
+    "flexatt_bwd_split",
     "flexatt_bwd_dkdv_ds",
     "flexatt_bwd_dq_ds",
     "flexatt_status_string",
@@ -113,6 +116,7 @@ def load() -> ctypes.CDLL:
         "flexatt_bwd_dkdv": [pr, T, T, T, T, fp, fp, T, T, st],
         "flexatt_bwd": [pr, T, T, T, T, T, fp, fp, T, T, T, st],
         "flexatt_bwd_ws": [pr, T, T, T, T, T, fp, fp, T, T, T, fp, ctypes.c_size_t, st],
+        "flexatt_bwd_split": [pr, T, T, T, T, T, fp, fp, T, T, T, fp, ctypes.c_size_t, st],
         "flexatt_bwd_dkdv_ds": [pr, T, T, T, T, fp, fp, T, T, fp, ctypes.c_size_t, st],
         "flexatt_bwd_dq_ds": [pr, T, fp, ctypes.c_size_t, T, st],
     }
@@ -120,13 +124,15 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.argtypes = args
         fn.restype = ctypes.c_int
-    for name in ("flexatt_fwd_decode_workspace", "flexatt_fwd_split_workspace", "flexatt_bwd_workspace"):
+    for name in ("flexatt_fwd_decode_workspace", "flexatt_fwd_split_workspace", "flexatt_bwd_workspace",
+                 "flexatt_bwd_split_workspace"):
         getattr(lib, name).argtypes = [pr]
         getattr(lib, name).restype = ctypes.c_size_t
     lib.flexatt_bwd_workspace_limited.argtypes = [pr, ctypes.c_size_t]
     lib.flexatt_bwd_workspace_limited.restype = ctypes.c_size_t
-    lib.flexatt_bwd_prefers_staging.argtypes = [pr]
-    lib.flexatt_bwd_prefers_staging.restype = ctypes.c_int
+    for name in ("flexatt_bwd_prefers_staging", "flexatt_bwd_prefers_split"):
+        getattr(lib, name).argtypes = [pr]
+        getattr(lib, name).restype = ctypes.c_int
     lib.flexatt_status_string.argtypes = [ctypes.c_int]
     lib.flexatt_status_string.restype = ctypes.c_char_p
     lib.flexatt_abi_version.argtypes = []

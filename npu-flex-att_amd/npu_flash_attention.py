@@ -474,8 +474,17 @@ def _backward_into(query, key, value, out, lse, grad_out, DQ, DK, DV, *, causal,
     lse = lse.to(torch.float32).contiguous()
     slopes = _alibi(alibi, Hq, query.device)
     p = _problem(q, k, scale, causal, sliding_window, soft_cap, slopes, masks)
-    ws_bytes = _staged_workspace_bytes(lib, p, query.device)
+    split = ds_staging_enabled and ds_staging_auto and lib.flexatt_bwd_prefers_split(p)
+    ws_bytes = lib.flexatt_bwd_split_workspace(p) if split else _staged_workspace_bytes(lib, p, query.device)
     with torch.cuda.device(query.device):
+        if split:
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device) if ws_bytes else None
+            st = lib.flexatt_bwd_split(p, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v), _lib.tensor(o),
+                                       _lib.tensor(do), lse.data_ptr(), delta.data_ptr(), _lib.tensor(DQ),
+                                       _lib.tensor(DK), _lib.tensor(DV), None if ws is None else ws.data_ptr(),
+                                       ws_bytes, _stream(query.device))
+            _lib.check(st, "flexatt_bwd_split")
+            return
         if ws_bytes:
             # the dK/dV kernel stages its dS in a workspace from torch's
             # caching allocator and dQ is formed from it

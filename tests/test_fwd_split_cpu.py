@@ -27,3 +27,25 @@ def test_split_rejections():
     assert lib.flexatt_fwd_split(p, t, t, t, t, FAKE, None, need, None) == -1
     assert lib.flexatt_fwd_split(p, t, t, t, t, None, FAKE, need, None) == -1
     assert lib.flexatt_fwd_split(p, t, t, t, t, FAKE, FAKE + 8, need, None) == -5
+
+
+@pytest.mark.parametrize("kw, code", [
+    (dict(head_dim=256), -6), (dict(dtype=L.F32), -6), (dict(block_map=FAKE, block_heads=1), -6), (dict(head_dim=48), -3),
+])
+def test_bwd_split_range(kw, code):
+    lib, p = L.load(), problem(**kw)
+    es = 4 if p.dtype == L.F32 else 2
+    t = tens(stride_s=p.head_dim, stride_h=64 * p.head_dim, stride_b=4 * 64 * p.head_dim)
+    assert es and lib.flexatt_bwd_prefers_split(p) == 0 and lib.flexatt_bwd_split_workspace(p) == 0
+    assert lib.flexatt_bwd_split(p, t, t, t, t, t, FAKE, FAKE, t, t, t, None, 0, None) == code
+
+
+def test_bwd_split_workspace_checks():
+    lib, p, t = L.load(), problem(heads_q=16, heads_kv=1, seqlen_q=640, seqlen_kv=640), tens(stride_h=640 * 64,
+                                                                                             stride_b=16 * 640 * 64)
+    need = lib.flexatt_bwd_split_workspace(p)
+    assert lib.flexatt_bwd_prefers_split(p) == 1 and need > 0  # the sums of two or more splits
+    args = (p, t, t, t, t, t, FAKE, FAKE, t, t, t)
+    assert lib.flexatt_bwd_split(*args, None, need, None) == -1
+    assert lib.flexatt_bwd_split(*args, FAKE, need - 1, None) == -1
+    assert lib.flexatt_bwd_split(*args, FAKE + 8, need, None) == -5
