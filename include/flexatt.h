@@ -254,7 +254,7 @@ int flexatt_bwd_ws(const flexatt_problem* p, const flexatt_tensor* q, const flex
  * Delta pass into `delta`, then dK/dV and dQ in one launch whose items split
  * their streams of tiles over the waves of a workgroup, and the long dK/dV
  * streams over several workgroups (fp32 sums in the workspace, added by one
- * more launch).  Range: fp16/bf16 at head_dim <= 128 without a block map (else
+ * more launch).  Range: head_dim <= 128 without a block map (else
  * FLEXATT_ERANGE).  `workspace`: flexatt_bwd_split_workspace(p) bytes, 16-byte
  * aligned, not zeroed, reusable once the call's work on `stream` is done; NULL
  * when that is 0.  Same results as flexatt_bwd up to fp32 summation order;

@@ -19,7 +19,7 @@ OUT_DIR = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libflexatt.so")
 HEAD_DIMS = (32, 64, 128, 256)
 PER_D_SOURCES = ("fwd_mfma.hip", "fwd_ws.hip", "fwd_split.hip", "bwd_mfma.hip", "bwd_kv.hip", "bwd_q.hip", "bwd_dq_ds.hip",
-                  "bwd_split.hip", "f32_mfma.hip")
+                  "bwd_split.hip", "f32_mfma.hip", "f32_split.hip")
 SINGLE_SOURCES = ("delta.hip", "doc_bounds.hip", "capi.hip")
 # Sources whose kernels load into registers through asm that the compiler
 # does not know is in flight (load16_async): a VGPR spill could store or

@@ -60,30 +60,6 @@ __device__ __forceinline__ int bsplit_swz(int r, int c) {
   else return swz_dual<CPR>(r, c);
 }
 
-// Sum over the waves of NA accumulators of DB blocks, in wave order: f(i, db,
-// quarter, values) for this wave's share of (accumulator i, block db, four of
-// its rows); every thread of the workgroup calls it.
-template <int NA, int DB, int NW, class F>
-__device__ __forceinline__ void combine_waves(char* smem, const f32x16 (&acc)[NA][DB], int wave, int lane, F f) {
-  float* x = (float*)smem;  // [NW][NA][DB][16][64]
-  __syncthreads();          // every wave is done with its tiles
-#pragma unroll
-  for (int i = 0; i < NA; ++i)
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) x[(((wave * NA + i) * DB + db) * 16 + e) * 64 + lane] = acc[i][db][e];
-  __syncthreads();
-  for (int u = wave; u < NA * DB * 4; u += NW) {
-    f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < NW; ++w)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) s[j] += x[(w * NA * DB * 16 + 4 * u + j) * 64 + lane];
-    f(u / (4 * DB), (u / 4) % DB, u % 4, s);
-  }
-}
-
 template <class T, int D, int NW, bool SOFTCAP, bool ALIBI>
 __global__ __launch_bounds__(NW * 64) void bwd_split_kernel(BwdSplitArgs a) {
   using C = BSplitCfg<D, NW>;

@@ -179,7 +179,7 @@ DecodePlan decode_plan(const flexatt_problem* p) {
   return d;
 }
 const DecodeLauncher kSplit[3][4] = {
-    {nullptr, nullptr, nullptr, nullptr},
+    {fwd_split_f32_d32, fwd_split_f32_d64, fwd_split_f32_d128, nullptr},  // one workgroup per row tile only
     {fwd_split_f16_d32, fwd_split_f16_d64, fwd_split_f16_d128, fwd_split_f16_d256},
     {fwd_split_bf16_d32, fwd_split_bf16_d64, fwd_split_bf16_d128, fwd_split_bf16_d256},
 };
@@ -315,8 +315,15 @@ int64_t attended_pairs(const flexatt_problem* p) {
 // chain is long enough to pay for the larger combine: H=2 D=64 S=2048 14.0 ->
 // 10.7, Hq=8 Hkv=2 D=128 S=2048 causal 27.2 -> 23.1 but non-causal 31.0 -> 34.4,
 // S=512 8.1 -> 8.9.
+// fp32 (f32_split.hip, four waves): an estimate in us of the split workgroups'
+// chain, or of the chip's time per 1024 tile pairs when they fill it, against
+// the regular kernel's chain (which eight waves of 256 rows walk together).
+// Measured, regular -> split: D = 128 Hq=8 S=1024 273 -> 52, B=2 S=2048 551 -> 217,
+// S=4096 non-causal 1126 -> 753; D = 64 H=2 S=2048 318 -> 55; D = 32 H=8 S=2048 204
+// -> 43.  The estimate of a full chip (5.9 us per 1024 pairs at D = 128, the
+// regular kernel 4.5) keeps large problems on the regular kernel.
 int split_waves(const flexatt_problem* p) {
-  if (!is_16bit(p) || p->block_map) return 0;
+  if (p->block_map || !kSplit[p->dtype][head_index(p->head_dim)]) return 0;
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const int64_t G = p->heads_q / p->heads_kv, groups = (int64_t)p->batch * p->heads_kv;
   const int64_t wgs = groups * ((G * p->seqlen_q + 31) / 32);
@@ -327,6 +334,12 @@ int split_waves(const flexatt_problem* p) {
   }
   const int64_t chain = (keys + 31) / 32;
   const int64_t units = groups * G * attended_pairs(p) / (32 * 32);
+  if (p->dtype == FLEXATT_F32) {
+    constexpr double tile[3] = {1.9, 3.2, 5.85}, unit[3] = {1.7, 2.9, 5.9}, other[3] = {3.2, 5.0, 8.4};
+    const int d = head_index(p->head_dim);
+    const double c = tile[d] * chain / 4, w = unit[d] * units / 1024;
+    return 5 + (c > w ? c : w) < 6 + other[d] * chain ? 4 : 0;
+  }
   if (p->head_dim == 256) return wgs <= cus ? 4 : 0;
   // (an eighth above the measured points, whose causal pairs are just over half)
   const int64_t load = 8 * units / (cus * chain);  // in eighths
@@ -652,7 +665,7 @@ int flexatt_bwd(const flexatt_problem* p, const flexatt_tensor* q, const flexatt
 
 namespace {
 const BwdSplitLauncher kBwdSplit[3][4] = {
-    {nullptr, nullptr, nullptr, nullptr},
+    {bwd_split_f32_d32, bwd_split_f32_d64, bwd_split_f32_d128, nullptr},
     {bwd_split_f16_d32, bwd_split_f16_d64, bwd_split_f16_d128, nullptr},
     {bwd_split_bf16_d32, bwd_split_bf16_d64, bwd_split_bf16_d128, nullptr},
 };
@@ -676,16 +689,24 @@ struct BwdSplitPlan {
   int nsplit, nw;
   size_t bytes;
 };
+// fp32 (four waves; 30 shapes): D = 128 10 us a tile and wave, 19.5 us per 1024
+// pairs (the other backward 11 once it fills the chip, which its estimate, a
+// chain, does not count, so that large problems stay with it).  Other -> split:
+// Hq=8 Hkv=2 S=1000 D=128 1264 -> 108 (4 x 4), H=2 S=2048 D=64 480 -> 93 (4 x 1).
 struct BwdSplitCost {
   double tile4, tile8, base4, base8, unit, wg4, wg8, other, other_kv, other_q;
 };
-constexpr BwdSplitCost kBwdSplitCost[3] = {
-    {0.8, 1.0, 6.0, 7.0, 1.0, 5.0, 10.0, 16.0, 0.65, 0.6},   // D = 32
-    {1.2, 1.4, 7.0, 8.5, 1.4, 8.0, 14.0, 14.0, 0.62, 0.4},   // 64
-    {1.6, 0.0, 9.0, 0.0, 2.8, 20.0, 0.0, 20.0, 0.95, 0.9},   // 128 (four waves only)
+constexpr BwdSplitCost kBwdSplitCost[2][3] = {
+    {{0.8, 1.0, 6.0, 7.0, 1.0, 5.0, 10.0, 16.0, 0.65, 0.6},    // fp16/bf16, D = 32
+     {1.2, 1.4, 7.0, 8.5, 1.4, 8.0, 14.0, 14.0, 0.62, 0.4},    // 64
+     {1.6, 0.0, 9.0, 0.0, 2.8, 20.0, 0.0, 20.0, 0.95, 0.9}},   // 128 (four waves only)
+    {{3.5, 0.0, 7.0, 0.0, 5.5, 8.0, 0.0, 10.0, 3.3, 1.2},      // fp32, D = 32
+     {5.7, 0.0, 8.0, 0.0, 9.0, 8.0, 0.0, 10.0, 5.3, 1.9},      // 64
+     {10.0, 0.0, 10.0, 0.0, 19.5, 10.0, 0.0, 10.0, 9.2, 4.0}}, // 128
 };
 BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
-  const BwdSplitCost& c = kBwdSplitCost[head_index(p->head_dim)];
+  const bool f32 = p->dtype == FLEXATT_F32;
+  const BwdSplitCost& c = kBwdSplitCost[f32][head_index(p->head_dim)];
   const double G = p->heads_q / p->heads_kv, groups = (double)p->batch * p->heads_kv;
   const int64_t nqt = (p->seqlen_q + 31) / 32, nkt = (p->seqlen_kv + 31) / 32;
   int64_t lq = nqt, lk = nkt;  // longest streams: query tiles of a KV item, key tiles of a Q item
@@ -700,7 +721,7 @@ BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
   const double part = 2.0 * sizeof(float) * groups * p->seqlen_kv * p->head_dim;  // bytes of one split's sums
   double best = 1e30;
   BwdSplitPlan r{false, 1, 4, 0};
-  for (int nw = 4; nw <= (p->head_dim < 128 ? 8 : 4); nw += 4)
+  for (int nw = 4; nw <= (p->head_dim < 128 && !f32 ? 8 : 4); nw += 4)
     for (int ns = 1; ns <= 8; ns *= 2) {
       const double t = nw == 8 ? c.tile8 : c.tile4, base = nw == 8 ? c.base8 : c.base4;
       const double wgs = groups * (double)(nkt * ns + nrt) / 1024;

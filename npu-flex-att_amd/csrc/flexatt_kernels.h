@@ -122,6 +122,14 @@ hipError_t bwd_split_f16_d64(const BwdSplitArgs&, hipStream_t);
 hipError_t bwd_split_bf16_d128(const BwdSplitArgs&, hipStream_t);
 hipError_t bwd_split_f16_d128(const BwdSplitArgs&, hipStream_t);
 
+// The same two for fp32 inputs (f32_split.hip; the forward with one split), D <= 128.
+hipError_t fwd_split_f32_d32(const DecodeArgs&, hipStream_t);
+hipError_t bwd_split_f32_d32(const BwdSplitArgs&, hipStream_t);
+hipError_t fwd_split_f32_d64(const DecodeArgs&, hipStream_t);
+hipError_t bwd_split_f32_d64(const BwdSplitArgs&, hipStream_t);
+hipError_t fwd_split_f32_d128(const DecodeArgs&, hipStream_t);
+hipError_t bwd_split_f32_d128(const BwdSplitArgs&, hipStream_t);
+
 // dK/dV as a KV-stationary tile stream (bwd_kv.hip), D = 64, 128 and 256.
 hipError_t bwd_kv_bf16_d128(const BwdArgs&, hipStream_t);
 hipError_t bwd_kv_f16_d128(const BwdArgs&, hipStream_t);

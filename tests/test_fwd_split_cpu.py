@@ -30,13 +30,12 @@ def test_split_rejections():
 
 
 @pytest.mark.parametrize("kw, code", [
-    (dict(head_dim=256), -6), (dict(dtype=L.F32), -6), (dict(block_map=FAKE, block_heads=1), -6), (dict(head_dim=48), -3),
+    (dict(head_dim=256), -6), (dict(dtype=L.F32, head_dim=256), -6), (dict(block_map=FAKE, block_heads=1), -6), (dict(head_dim=48), -3),
 ])
 def test_bwd_split_range(kw, code):
     lib, p = L.load(), problem(**kw)
-    es = 4 if p.dtype == L.F32 else 2
     t = tens(stride_s=p.head_dim, stride_h=64 * p.head_dim, stride_b=4 * 64 * p.head_dim)
-    assert es and lib.flexatt_bwd_prefers_split(p) == 0 and lib.flexatt_bwd_split_workspace(p) == 0
+    assert lib.flexatt_bwd_prefers_split(p) == 0 and lib.flexatt_bwd_split_workspace(p) == 0
     assert lib.flexatt_bwd_split(p, t, t, t, t, t, FAKE, FAKE, t, t, t, None, 0, None) == code
 
 

@@ -33,6 +33,10 @@ SHAPES = [
     (torch.bfloat16, 128, 1, 6, 2, 95, 97),
     (torch.float16, 128, 1, 8, 1, 420, 420),   # several workgroups a stream
     (torch.bfloat16, 128, 2, 1, 1, 32, 1),
+    (torch.float32, 32, 1, 3, 1, 70, 70),
+    (torch.float32, 64, 2, 2, 2, 1, 33),
+    (torch.float32, 128, 1, 6, 2, 95, 97),
+    (torch.float32, 128, 1, 8, 1, 260, 260),   # several workgroups a stream
 ]
 
 
@@ -82,7 +86,7 @@ def test_split_matches_oracle(gpu_device, shape, flags):
 
 
 @pytest.mark.parametrize("flags", list(FLAGS))
-@pytest.mark.parametrize("shape", SHAPES[:6],
+@pytest.mark.parametrize("shape", SHAPES[:6] + SHAPES[8:11],
                          ids=lambda s: f"d{s[1]}_b{s[2]}_h{s[3]}_{s[4]}_{s[5]}x{s[6]}")
 def test_other_backward_at_the_same_sizes(gpu_device, monkeypatch, shape, flags):
     if flags == "cap_wide_window":

@@ -31,7 +31,12 @@ SHAPES = [
     (torch.bfloat16, 128, 1, 6, 2, 95, 97),
     (torch.float16, 128, 1, 2, 1, 2049, 2049),  # eight waves
     (torch.bfloat16, 256, 1, 4, 2, 130, 160),
+    (torch.float32, 32, 1, 3, 1, 70, 70),
+    (torch.float32, 64, 1, 2, 2, 1, 33),
+    (torch.float32, 128, 1, 6, 2, 95, 97),
     # a full grid: the regular forward
+    (torch.float32, 32, 48, 16, 8, 100, 100),
+    (torch.float32, 128, 48, 16, 8, 60, 60),
     (torch.bfloat16, 64, 64, 32, 8, 150, 150),
     (torch.float16, 128, 24, 16, 8, 150, 150),
 ]
