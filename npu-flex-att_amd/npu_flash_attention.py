@@ -35,6 +35,7 @@ DESIGN.md:374 list them as unsupported or future work), on every entry point:
 """
 from __future__ import annotations
 
+import contextlib
 import math
 from dataclasses import dataclass
 from typing import Optional
@@ -97,10 +98,16 @@ def _kernel_ready(t: torch.Tensor) -> bool:
 
 
 def _prepare(t: torch.Tensor) -> torch.Tensor:
+    # (a contiguous tensor on a 16-byte boundary is ready at every head dim,
+    # without the look at each stride, 1 us a tensor)
+    if t.is_contiguous() and t.data_ptr() % 16 == 0:
+        return t
     return t if _kernel_ready(t) else t.contiguous()
 
 
 def _check_device_dtype(name_tensors, dtype):
+    if all([isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype for _, t in name_tensors]):
+        return
     for name, t in name_tensors:
         if not isinstance(t, torch.Tensor):
             raise RuntimeError(f"{name} must be a torch.Tensor")
@@ -129,18 +136,14 @@ def _problem(query, key, scale, causal, sliding_window, soft_cap, alibi, masks=N
         raise RuntimeError(f"unsupported dtype {query.dtype} (expected float32, float16 or bfloat16)")
     if D not in _HEAD_DIMS:
         raise RuntimeError(f"unsupported head dim {D} (expected one of {_HEAD_DIMS})")
-    p = _lib.Problem()
-    p.dtype = _DTYPES[query.dtype]
-    p.batch, p.heads_q, p.heads_kv, p.seqlen_q, p.seqlen_kv, p.head_dim = B, Hq, Hkv, Sq, Sk, D
-    p.scale = float(scale)
     if masks is not None:
         causal = masks.causal
-    p.causal = 1 if causal else 0
     # The reference enables a primitive only for a positive value
     # (npu_flash_attention.py:70, :648).
-    p.sliding_window = int(sliding_window) if sliding_window and sliding_window > 0 else 0
-    p.soft_cap = float(soft_cap) if soft_cap and soft_cap > 0.0 else 0.0
-    p.alibi_slopes = alibi.data_ptr() if alibi is not None else None
+    p = _lib.Problem(_DTYPES[query.dtype], B, Hq, Hkv, Sq, Sk, D, float(scale), 1 if causal else 0,
+                     int(sliding_window) if sliding_window and sliding_window > 0 else 0,
+                     float(soft_cap) if soft_cap and soft_cap > 0.0 else 0.0,
+                     alibi.data_ptr() if alibi is not None else None)
     if masks is not None:
         p.doc_bounds = masks.rows.data_ptr() if masks.rows is not None else None
         p.col_bounds = masks.cols.data_ptr() if masks.cols is not None else None
@@ -176,7 +179,7 @@ def _doc_bounds(document_ids, B, Sq, Sk, device, native=False):
     if native and ids.is_cuda and ids.numel() > 0:
         ids = ids.contiguous()
         bounds = torch.empty(B, S, 2, dtype=torch.int32, device=ids.device)
-        with torch.cuda.device(ids.device):
+        with _device_guard(ids.device):
             st = _lib.load().flexatt_document_bounds(ids.data_ptr(), ids.element_size(), B, S, bounds.data_ptr(),
                                                      _stream(ids.device))
         _lib.check(st, "flexatt_document_bounds")
@@ -250,7 +253,7 @@ def _block_map(block_mask, B, Hq, Sq, Sk, device):
         if m.dim() != 4 or m.shape[2] != nq or m.shape[3] != nk:
             raise RuntimeError(f"a dense block_mask must be [B|1, Hq|1, {nq}, {nk}] (blocks of {_BLOCK}), "
                                f"got {tuple(m.shape)}")
-        m = m != 0
+        m = m.view(torch.uint8) if m.dtype == torch.bool else m != 0  # (a bool is one byte, 0 or 1)
     else:
         if isinstance(block_mask, (tuple, list)) and len(block_mask) == 2:
             parts = [tuple(block_mask)]
@@ -299,7 +302,15 @@ def _masks(causal, document_ids, prefix_len, block_mask, B, Hq, Sq, Sk, device, 
 
 
 def _stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def _device_guard(device):
+    """The kernels run on the current device: make it the tensors' own."""
+    return _SAME_DEVICE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 # ------------------------------------------------------------- forward (L2) --
@@ -340,7 +351,7 @@ def npu_flash_attention_forward(
         scale = 1.0 / math.sqrt(D)
 
     O = torch.empty_like(query)
-    if not _kernel_ready(O):
+    if not O.is_contiguous() and not _kernel_ready(O):
         O = torch.empty(query.shape, dtype=query.dtype, device=query.device)
     LSE = torch.empty(B, Hq, Sq, device=query.device, dtype=torch.float32)
     masks = _masks(causal, document_ids, prefix_len, block_mask, B, Hq, Sq, Sk, query.device, native=True)
@@ -365,7 +376,7 @@ def _forward_into(query, key, value, O, LSE, *, causal, sliding_window, alibi, s
     # Few query rows per KV head (decoding): the split-KV kernels, with their
     # partial results in a workspace from torch's caching allocator.
     ws_bytes = lib.flexatt_fwd_split_workspace(p) if decode_enabled else 0
-    with torch.cuda.device(query.device):
+    with _device_guard(query.device):
         if ws_bytes:
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device)
             st = lib.flexatt_fwd_split(p, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v), _lib.tensor(O),
@@ -415,7 +426,7 @@ def npu_flash_attention_backward(
         scale = 1.0 / math.sqrt(D)
 
     DQ = torch.empty_like(query)
-    if not _kernel_ready(DQ):
+    if not DQ.is_contiguous() and not _kernel_ready(DQ):
         DQ = torch.empty(query.shape, dtype=query.dtype, device=query.device)
     DK = torch.empty(B, Hkv, Sk, D, device=key.device, dtype=key.dtype)
     DV = torch.empty(B, Hkv, Sk, D, device=value.device, dtype=value.dtype)
@@ -471,12 +482,13 @@ def _backward_into(query, key, value, out, lse, grad_out, DQ, DK, DV, *, causal,
     lib = _lib.load()
     q, k, v = _prepare(query), _prepare(key), _prepare(value)
     o, do = _prepare(out), _prepare(grad_out)
-    lse = lse.to(torch.float32).contiguous()
+    if lse.dtype != torch.float32 or not lse.is_contiguous():
+        lse = lse.to(torch.float32).contiguous()
     slopes = _alibi(alibi, Hq, query.device)
     p = _problem(q, k, scale, causal, sliding_window, soft_cap, slopes, masks)
     split = ds_staging_enabled and ds_staging_auto and lib.flexatt_bwd_prefers_split(p)
     ws_bytes = lib.flexatt_bwd_split_workspace(p) if split else _staged_workspace_bytes(lib, p, query.device)
-    with torch.cuda.device(query.device):
+    with _device_guard(query.device):
         if split:
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device) if ws_bytes else None
             st = lib.flexatt_bwd_split(p, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v), _lib.tensor(o),
@@ -523,15 +535,14 @@ class NPUFlexAttention(torch.autograd.Function):
         ctx.document_ids = document_ids
         ctx.prefix_len = prefix_len
         ctx.block_mask = block_mask
-        with torch.no_grad():
-            out, lse = npu_flash_attention_forward(
-                query, key, value,
-                causal=causal, sliding_window=sliding_window,
-                alibi_slope=alibi_slope, scale=scale,
-                block_m=block_m, block_n=block_n, return_lse=True,
-                soft_cap=soft_cap, document_ids=document_ids,
-                prefix_len=prefix_len, block_mask=block_mask,
-            )
+        out, lse = npu_flash_attention_forward(  # (autograd runs this method without grad)
+            query, key, value,
+            causal=causal, sliding_window=sliding_window,
+            alibi_slope=alibi_slope, scale=scale,
+            block_m=block_m, block_n=block_n, return_lse=True,
+            soft_cap=soft_cap, document_ids=document_ids,
+            prefix_len=prefix_len, block_mask=block_mask,
+        )
         ctx.save_for_backward(query, key, value, lse, out)
         return out
 
