@@ -267,6 +267,13 @@ int flexatt_bwd_split(const flexatt_problem* p, const flexatt_tensor* q, const f
                       const float* lse, float* delta, const flexatt_tensor* dq, const flexatt_tensor* dk,
                       const flexatt_tensor* dv, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Bytes worth adding to a whole-band workspace of flexatt_bwd_ws (after the
+ * queue counters): where a KV block per CU leaves the dK/dV launch waiting for
+ * its longest blocks, flexatt_bwd_ws then shares each block's query tiles
+ * between workgroups and adds their fp32 sums from there, the same results up
+ * to summation order.  0: nothing to gain. */
+size_t flexatt_bwd_ws_parts_bytes(const flexatt_problem* p);
+
 /* The two kernels of flexatt_bwd_ws on their own (FLEXATT_ERANGE outside
  * its range).  flexatt_bwd_dkdv_ds replaces the flash_attn_bwd_dkdv_kernel
  * launch and the group sum (npu_flash_attention.py:714-737) and also fills

@@ -105,8 +105,8 @@ struct KvCfg {
 // slower, 570 -> 580 us at bf16 B=2 Hq=32 Hkv=8 S=4096 causal.)
 // The tile stream of one work item: KV block kb of (b, hkv) = bh, walked as
 // workgroup slot `slot` (which sets the walk direction), in the LDS at smem.
-template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, int PASS, bool BLK, bool DOC, int TPS = 1>
-__device__ __forceinline__ void kv_tile_stream(const BwdArgs& a, char* smem, int slot, int kb, int bh) {
+template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, int PASS, bool BLK, bool DOC, bool PART, int TPS = 1>
+__device__ __forceinline__ void kv_tile_stream(const BwdArgs& a, char* smem, int slot, int kb, int bh, int part) {
   using C = KvCfg<D, TPS>;
   static_assert(TPS == 1 || (TPS == 2 && PASS == 0 && !BLK && D == 128), "two tiles per step: D = 128, no block maps");
   static_assert(C::DB == 2 * C::KC / 4 && (D == 64 || D == 128 || D == 256), "head dims 64, 128, 256");
@@ -151,11 +151,14 @@ __device__ __forceinline__ void kv_tile_stream(const BwdArgs& a, char* smem, int
     q_lo = __builtin_amdgcn_readfirstlane(max(q_lo, l));
     q_hi = __builtin_amdgcn_readfirstlane(min(q_hi, h));
   }
-  const int qt_lo = q_lo / C::BM;
   // (interval masks: by whole tiles, as the dQ kernel counts them, ds_doc_range)
-  const int nqt = DOC            ? max((q_hi + C::BM - 1) / C::BM - qt_lo, 0)
-                  : q_hi > q_lo ? (q_hi + C::BM - 1) / C::BM - qt_lo
-                                : 0;
+  const int qt_first = q_lo / C::BM;
+  const int nqt_all = DOC            ? max((q_hi + C::BM - 1) / C::BM - qt_first, 0)
+                      : q_hi > q_lo ? (q_hi + C::BM - 1) / C::BM - qt_first
+                                    : 0;
+  // this workgroup's share of them
+  const int qt_lo = PART ? qt_first + nqt_all * part / a.nparts : qt_first;
+  const int nqt = PART ? nqt_all * (part + 1) / a.nparts - nqt_all * part / a.nparts : nqt_all;
   int ntile = p.G * nqt;
   // Tile order: the G heads of a query tile consecutively; the first round
   // of workgroups (one per CU) walks the query tiles from the last one down,
@@ -958,6 +961,24 @@ __device__ __forceinline__ void kv_tile_stream(const BwdArgs& a, char* smem, int
     }  // TPS == 1
     wait_vmcnt<0>();  // redundant copies in flight must land before the workgroup ends
 
+    if constexpr (PART) {  // this share's sums in fp32: [part][dK, dV][B * Hkv * Skv][D]
+      if (my_kv < p.Skv) {
+        const int64_t n = (int64_t)p.B * p.Hkv * p.Skv * D;
+        float* o = a.part + 2 * part * n + ((int64_t)bh * p.Skv + my_kv) * D + 4 * h;
+#pragma unroll
+        for (int db = 0; db < C::DB; ++db)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if constexpr (DOK)
+              *(f32x4*)(o + 32 * db + 8 * i) =
+                  f32x4{dk[db][4 * i], dk[db][4 * i + 1], dk[db][4 * i + 2], dk[db][4 * i + 3]} * p.scale;
+            if constexpr (DOV)
+              *(f32x4*)(o + n + 32 * db + 8 * i) =
+                  f32x4{dv[db][4 * i], dv[db][4 * i + 1], dv[db][4 * i + 2], dv[db][4 * i + 3]};
+          }
+      }
+      return;
+    }
     // dK = scale * sum dS^T Q, dV = sum P^T dO; lane = KV row.
     if (my_kv < p.Skv) {
       T* kq = (T*)a.dk.data + b * a.dk.sb + hk * a.dk.sh + (int64_t)my_kv * a.dk.ss + 4 * h;
@@ -981,11 +1002,11 @@ __device__ __forceinline__ void kv_tile_stream(const BwdArgs& a, char* smem, int
 // D = 64 and 128 (PASS 0).  Work item: (b, hkv, KV block), blocks of
 // one (b, hkv) consecutive so that they share an XCD (and its L2) and heavy /
 // light causal blocks interleave; block 0 has the longest causal band.
-template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, int PASS, bool BLK, bool DOC, int TPS = 1>
+template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, int PASS, bool BLK, bool DOC, bool PART, int TPS = 1>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KvCfg<D>::WPE, KvCfg<D>::WPE)))
 void bwd_kv_kernel(BwdArgs a) {
   __shared__ __attribute__((aligned(1024))) char smem[KvCfg<D, TPS>::LDSB];
-  const int nkb = a.ntiles;
+  const int nkb = PART ? a.ntiles * a.nparts : a.ntiles;  // (kb counts a KV block's parts as well)
   const int slot = queue_slot(a.queue, a.nstatic);
   if (slot >= (int)gridDim.x) return;  // (a counter that was not cleared)
   int kb, bh;
@@ -994,7 +1015,12 @@ void bwd_kv_kernel(BwdArgs a) {
     kb = w % nkb;
     bh = w / nkb;
   }
-  kv_tile_stream<T, D, SOFTCAP, ALIBI, DS, PASS, BLK, DOC, TPS>(a, smem, slot, kb, bh);
+  int part = 0;
+  if constexpr (PART) {
+    part = kb % a.nparts;
+    kb /= a.nparts;
+  }
+  kv_tile_stream<T, D, SOFTCAP, ALIBI, DS, PASS, BLK, DOC, PART, TPS>(a, smem, slot, kb, bh, part);
 }
 
 // D = 256: the dV pass (PASS 1) and the dK pass (PASS 2) of every KV block in
@@ -1005,12 +1031,12 @@ void bwd_kv_kernel(BwdArgs a) {
 // (at config 4, 132 query tiles then 128 .. 4 per CU, against 99 on average).
 // Item k of a group: KV block k / 2, the dK pass for even k (the longer of the
 // two per tile: dP MFMAs and the staged dS stores) and the dV pass for odd k.
-template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, bool BLK, bool DOC>
+template <class T, int D, bool SOFTCAP, bool ALIBI, bool DS, bool BLK, bool DOC, bool PART>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KvCfg<D>::WPE, KvCfg<D>::WPE)))
 void bwd_kv_passes_kernel(BwdArgs a) {
   static_assert(KvCfg<D>::PASSES, "two passes at D = 256 only");
   __shared__ __attribute__((aligned(1024))) char smem[KvCfg<D>::LDSB];
-  const int nit = 2 * a.ntiles;  // items per (b, hkv)
+  const int nit = 2 * a.ntiles * (PART ? a.nparts : 1);  // items per (b, hkv)
   const int slot = queue_slot(a.queue, a.nstatic);
   if (slot >= (int)gridDim.x) return;  // (a counter that was not cleared)
   int k, bh;
@@ -1019,8 +1045,14 @@ void bwd_kv_passes_kernel(BwdArgs a) {
     k = w % nit;
     bh = w / nit;
   }
-  if ((k & 1) == 0) kv_tile_stream<T, D, SOFTCAP, ALIBI, DS, 2, BLK, DOC>(a, smem, slot, k >> 1, bh);
-  else kv_tile_stream<T, D, SOFTCAP, ALIBI, false, 1, BLK, DOC>(a, smem, slot, k >> 1, bh);
+  if constexpr (PART) {
+    const int kb = (k >> 1) / a.nparts, part = (k >> 1) % a.nparts;
+    if ((k & 1) == 0) kv_tile_stream<T, D, SOFTCAP, ALIBI, DS, 2, BLK, DOC, true>(a, smem, slot, kb, bh, part);
+    else kv_tile_stream<T, D, SOFTCAP, ALIBI, false, 1, BLK, DOC, true>(a, smem, slot, kb, bh, part);
+  } else {
+    if ((k & 1) == 0) kv_tile_stream<T, D, SOFTCAP, ALIBI, DS, 2, BLK, DOC, false>(a, smem, slot, k >> 1, bh, 0);
+    else kv_tile_stream<T, D, SOFTCAP, ALIBI, false, 1, BLK, DOC, false>(a, smem, slot, k >> 1, bh, 0);
+  }
 }
 
 #ifndef FLEXATT_KV_TPS
@@ -1033,7 +1065,7 @@ hipError_t launch_kv(const BwdArgs& a, hipStream_t st) {
   static_assert(C::BKV == kDsKB && C::BM == kDsQT, "staged dS units are one tile by one KV block");
   BwdArgs x = a;
   x.ntiles = (a.p.Skv + C::BKV - 1) / C::BKV;
-  const int items = x.ntiles * a.p.B * a.p.Hkv;
+  const int items = x.ntiles * a.p.B * a.p.Hkv * (DS ? a.nparts : 1);
   const dim3 block(C::NW * 64);
   // block-sparse maps: the walk list of live query tiles in dynamic LDS
   // (when it fits beside the tile stages; otherwise removed tiles are walked
@@ -1041,29 +1073,38 @@ hipError_t launch_kv(const BwdArgs& a, hipStream_t st) {
   const size_t list = 2 * (size_t)((a.p.Sq + C::BM - 1) / C::BM + 2);
   const bool blk = a.p.blk && C::LDSB + list <= 160 * 1024;
   const size_t dyn = blk ? list : 0;
-  auto go = [&](auto sc, auto al, auto bl, auto doc) {
+  auto go = [&](auto sc, auto al, auto bl, auto doc, auto pt) {
     constexpr bool SC = decltype(sc)::value, AL = decltype(al)::value, BL = decltype(bl)::value,
-                   DOC = decltype(doc)::value;
+                   DOC = decltype(doc)::value, PT = decltype(pt)::value;
     if constexpr (C::PASSES) {  // both passes' items in one launch
-      hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, SC, AL, DS, BL, DOC>), dim3(2 * items), block, dyn, st, x);
+      hipLaunchKernelGGL((bwd_kv_passes_kernel<T, D, SC, AL, DS, BL, DOC, PT>), dim3(2 * items), block, dyn, st, x);
     } else {
       if constexpr (D == 128 && !BL && FLEXATT_KV_TPS == 2) {
         if (!a.p.blk) {
-          hipLaunchKernelGGL((bwd_kv_kernel<T, D, SC, AL, DS, 0, BL, DOC, FLEXATT_KV_TPS>), dim3(items), block, dyn, st,
-                             x);
+          hipLaunchKernelGGL((bwd_kv_kernel<T, D, SC, AL, DS, 0, BL, DOC, PT, FLEXATT_KV_TPS>), dim3(items), block, dyn,
+                             st, x);
           return;
         }
       }
-      hipLaunchKernelGGL((bwd_kv_kernel<T, D, SC, AL, DS, 0, BL, DOC>), dim3(items), block, dyn, st, x);
+      hipLaunchKernelGGL((bwd_kv_kernel<T, D, SC, AL, DS, 0, BL, DOC, PT>), dim3(items), block, dyn, st, x);
     }
   };
   using std::false_type;
   using std::true_type;
+  auto parts = [&](auto sc, auto al, auto bl, auto doc) {
+    if constexpr (DS) {
+      if (a.nparts > 1) {
+        go(sc, al, bl, doc, true_type{});
+        return;
+      }
+    }
+    go(sc, al, bl, doc, false_type{});
+  };
   auto masks = [&](auto sc, auto al) {
-    if (blk && a.p.docc) go(sc, al, true_type{}, true_type{});
-    else if (blk) go(sc, al, true_type{}, false_type{});
-    else if (a.p.docc) go(sc, al, false_type{}, true_type{});
-    else go(sc, al, false_type{}, false_type{});
+    if (blk && a.p.docc) parts(sc, al, true_type{}, true_type{});
+    else if (blk) parts(sc, al, true_type{}, false_type{});
+    else if (a.p.docc) parts(sc, al, false_type{}, true_type{});
+    else parts(sc, al, false_type{}, false_type{});
   };
   const bool sc = a.p.cap > 0.f, al = a.p.alibi != nullptr;
   if (sc && al) masks(true_type{}, true_type{});

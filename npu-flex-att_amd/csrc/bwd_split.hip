@@ -39,6 +39,38 @@
 
 namespace flexatt {
 
+// dK and dV from the splits' sums, in split order: four columns per thread.
+template <class T, int D>
+__global__ __launch_bounds__(256) void bwd_split_sum_kernel(BwdSplitArgs a) {
+  const Shape& p = a.p;
+  const int64_t n = (int64_t)p.B * p.Hkv * p.Skv * D;
+  const int64_t x = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
+  if (x >= 2 * n) return;
+  const int which = x >= n;
+  const int64_t y = x - which * n, row = y / D, bh = row / p.Skv;
+  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < a.nsplit; ++s) v += *(const f32x4*)(a.part + (2 * s + which) * n + y);
+  const MutView& t = which ? a.dv : a.dk;
+  T* dst = (T*)t.data + bh / p.Hkv * t.sb + bh % p.Hkv * t.sh + row % p.Skv * t.ss + y % D;
+  st_global8(dst, pack4<T>(v[0], v[1], v[2], v[3]));
+}
+
+template <class T, int D>
+hipError_t launch_split_sum(const BwdSplitArgs& a, hipStream_t st) {
+  const int64_t n = 2 * (int64_t)a.p.B * a.p.Hkv * a.p.Skv * D / 4;
+  hipLaunchKernelGGL((bwd_split_sum_kernel<T, D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
+#define FLEXATT_CAT2(a, b) a##b
+#define FLEXATT_CAT(a, b) FLEXATT_CAT2(a, b)
+hipError_t FLEXATT_CAT(bwd_split_sum_bf16_d, FLEXATT_D)(const BwdSplitArgs& a, hipStream_t st) {
+  return launch_split_sum<__bf16, FLEXATT_D>(a, st);
+}
+hipError_t FLEXATT_CAT(bwd_split_sum_f16_d, FLEXATT_D)(const BwdSplitArgs& a, hipStream_t st) {
+  return launch_split_sum<_Float16, FLEXATT_D>(a, st);
+}
+
 #if FLEXATT_D <= 128
 
 template <int D, int NW>
@@ -324,22 +356,6 @@ __global__ __launch_bounds__(NW * 64) void bwd_split_kernel(BwdSplitArgs a) {
   }
 }
 
-// dK and dV from the splits' sums, in split order: four columns per thread.
-template <class T, int D>
-__global__ __launch_bounds__(256) void bwd_split_sum_kernel(BwdSplitArgs a) {
-  const Shape& p = a.p;
-  const int64_t n = (int64_t)p.B * p.Hkv * p.Skv * D;
-  const int64_t x = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
-  if (x >= 2 * n) return;
-  const int which = x >= n;
-  const int64_t y = x - which * n, row = y / D, bh = row / p.Skv;
-  f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < a.nsplit; ++s) v += *(const f32x4*)(a.part + (2 * s + which) * n + y);
-  const MutView& t = which ? a.dv : a.dk;
-  T* dst = (T*)t.data + bh / p.Hkv * t.sb + bh % p.Hkv * t.sh + row % p.Skv * t.ss + y % D;
-  st_global8(dst, pack4<T>(v[0], v[1], v[2], v[3]));
-}
-
 template <class T, int D, int NW>
 hipError_t launch_bwd_split(const BwdSplitArgs& a, hipStream_t st) {
   const dim3 grid(a.p.B * a.p.Hkv * (a.nkt * a.nsplit + a.nrt)), block(NW * 64);
@@ -349,10 +365,7 @@ hipError_t launch_bwd_split(const BwdSplitArgs& a, hipStream_t st) {
   else if (al) hipLaunchKernelGGL((bwd_split_kernel<T, D, NW, false, true>), grid, block, 0, st, a);
   else hipLaunchKernelGGL((bwd_split_kernel<T, D, NW, false, false>), grid, block, 0, st, a);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess || a.nsplit == 1) return e;
-  const int64_t n = 2 * (int64_t)a.p.B * a.p.Hkv * a.p.Skv * D / 4;
-  hipLaunchKernelGGL((bwd_split_sum_kernel<T, D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);
-  return hipGetLastError();
+  return e != hipSuccess || a.nsplit == 1 ? e : launch_split_sum<T, D>(a, st);
 }
 
 template <class T, int D>
@@ -366,8 +379,6 @@ hipError_t launch_bwd_split(const BwdSplitArgs& a, hipStream_t st) {
   return launch_bwd_split<T, D, 4>(x, st);
 }
 
-#define FLEXATT_CAT2(a, b) a##b
-#define FLEXATT_CAT(a, b) FLEXATT_CAT2(a, b)
 hipError_t FLEXATT_CAT(bwd_split_bf16_d, FLEXATT_D)(const BwdSplitArgs& a, hipStream_t st) {
   return launch_bwd_split<__bf16, FLEXATT_D>(a, st);
 }

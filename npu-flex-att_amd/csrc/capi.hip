@@ -370,6 +370,8 @@ int bwd_common(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_
   a.ds = nullptr;
   a.ds_head = 0;
   a.queue = nullptr;
+  a.part = nullptr;
+  a.nparts = 1;
   a.nstatic = cu_count() & ~7;  // the first round of workgroups (also sets the dK/dV walk direction)
   return FLEXATT_OK;
 }
@@ -664,6 +666,33 @@ int flexatt_bwd(const flexatt_problem* p, const flexatt_tensor* q, const flexatt
 }
 
 namespace {
+// Workgroups that share the query tiles of one KV block in the staged dK/dV
+// launch (fp16/bf16).  With one item per KV block and no more items than CUs the
+// launch lasts as long as its longest block, and under a causal mask the
+// average one is half as long: about two items per CU even that out
+// (longest first).  More cost their fp32 sums.  Backward, parts 1 / 2 / 3 / 4, us, D = 128
+// causal: Hq=32 Hkv=8 S=4096 604 / 501 / 515 / 523 (256 blocks), with half the blocks
+// masked away 477 / 345 / 351 / 362, S=3000 429 / 333 / 318 / 331 (192), S=2048 295 / 218 /
+// 194 / 194 (128), Hkv=16 S=4096 479 / 532 (512); non-causal, whose blocks are equally long
+// and fill one round: S=2048 300 / 246 / 282 / 265, S=4096 785 / 835; D = 64, two workgroups a
+// CU: half the blocks masked S=4096 416 / 311 / 285 / 272; D = 256, two passes a block:
+// Hq=16 S=1000 141 / 102 / 97 / 101, S=4096 565 / 582.
+int staged_parts(const flexatt_problem* p) {
+  if (!is_16bit(p) || p->head_dim == 32) return 1;
+  const int cus = cu_count() > 0 ? cu_count() : 256;
+  const int64_t items = (int64_t)p->batch * p->heads_kv * ((p->seqlen_kv + kDsKB - 1) / kDsKB) * (p->head_dim == 256 ? 2 : 1);
+  const int64_t slots = p->head_dim == 64 ? 2 * cus : cus;
+  // blocks equally long: no causal mask, or a window that most of them see whole
+  const bool uniform = !has_masks(p) && (!p->causal || (p->sliding_window > 0 && p->sliding_window <= p->seqlen_q / 4));
+  int64_t n = uniform ? slots / items : (2 * slots + items / 2) / items;
+  const int64_t most = (p->seqlen_q + 4 * kDsQT - 1) / (4 * kDsQT);  // at least about four query tiles each
+  if (n > most) n = most;
+  return (int)(n > 4 ? 4 : n < 1 ? 1 : n);
+}
+size_t part_bytes(const flexatt_problem* p, int nparts) {
+  return 2 * sizeof(float) * (size_t)nparts * p->batch * p->heads_kv * p->seqlen_kv * p->head_dim;
+}
+
 const BwdSplitLauncher kBwdSplit[3][4] = {
     {bwd_split_f32_d32, bwd_split_f32_d64, bwd_split_f32_d128, nullptr},
     {bwd_split_f16_d32, bwd_split_f16_d64, bwd_split_f16_d128, nullptr},
@@ -707,6 +736,7 @@ constexpr BwdSplitCost kBwdSplitCost[2][3] = {
 BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
   const bool f32 = p->dtype == FLEXATT_F32;
   const BwdSplitCost& c = kBwdSplitCost[f32][head_index(p->head_dim)];
+  const bool cap = p->soft_cap > 0.f;
   const double G = p->heads_q / p->heads_kv, groups = (double)p->batch * p->heads_kv;
   const int64_t nqt = (p->seqlen_q + 31) / 32, nkt = (p->seqlen_kv + 31) / 32;
   int64_t lq = nqt, lk = nkt;  // longest streams: query tiles of a KV item, key tiles of a Q item
@@ -726,7 +756,7 @@ BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
       const double t = nw == 8 ? c.tile8 : c.tile4, base = nw == 8 ? c.base8 : c.base4;
       const double wgs = groups * (double)(nkt * ns + nrt) / 1024;
       const double chain = t * (G * lq / ns > lk ? G * lq / ns : lk) / nw;
-      const double work = c.unit * units + (nw == 8 ? c.wg8 : c.wg4) * wgs;
+      const double work = c.unit * (cap ? 1.25 : 1.0) * units + (nw == 8 ? c.wg8 : c.wg4) * wgs;
       // the sums written and read back at about 8 TB/s (they stay in cache), and one more launch
       const double est = base + (chain > work ? chain : work) + (ns > 1 ? 4 + 2 * ns * part / 8e6 : 0);
       if (est < best) {
@@ -735,7 +765,15 @@ BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
         r.nw = nw;
       }
     }
-  r.faster = best < c.other + c.other_kv * G * lq + c.other_q * lk;
+  // the staged backward where it is preferred, its dK/dV streams shared by parts
+  const int np = flexatt_bwd_prefers_staging(p) ? staged_parts(p) : 1;
+  double other = c.other + c.other_kv * (cap ? 1.2 : 1.0) * G * lq / np + c.other_q * lk;
+  if (p->head_dim == 64 && cap && !f32) other = 20 + 1.22 * G * lq / np + c.other_q * lk;
+  if (np > 1) {
+    const double work = 25 + 1.75 * units;
+    other = (other > work ? other : work) + 8 + 2 * np * part / 8e6;
+  }
+  r.faster = best < other;
   if (r.nsplit > 1) r.bytes = (size_t)(part * r.nsplit);
   return r;
 }
@@ -809,9 +847,15 @@ size_t flexatt_bwd_workspace_limited(const flexatt_problem* p, size_t limit_byte
 }
 
 namespace {
+const BwdSplitLauncher kPartSum[3][4] = {
+    {nullptr, nullptr, nullptr, nullptr},
+    {bwd_split_sum_f16_d32, bwd_split_sum_f16_d64, bwd_split_sum_f16_d128, bwd_split_sum_f16_d256},
+    {bwd_split_sum_bf16_d32, bwd_split_sum_bf16_d64, bwd_split_sum_bf16_d128, bwd_split_sum_bf16_d256},
+};
 int run_dkdv_ds(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k, const flexatt_tensor* v,
                 const flexatt_tensor* dout, const float* lse, const float* delta, const flexatt_tensor* dk,
-                const flexatt_tensor* dv, void* workspace, size_t workspace_bytes, int* queue, void* stream) {
+                const flexatt_tensor* dv, void* workspace, size_t workspace_bytes, int* queue, float* part, int nparts,
+                void* stream) {
   BwdArgs a;
   FLEXATT_TRY(bwd_common(p, q, k, v, dout, lse, delta, a));
   FLEXATT_TRY(check_out_tensor(dk, p->dtype, p->batch, p->heads_kv, p->seqlen_kv, p->head_dim));
@@ -821,7 +865,17 @@ int run_dkdv_ds(const flexatt_problem* p, const flexatt_tensor* q, const flexatt
   a.dv = mview(dv);
   a.queue = queue;
   a.nstatic = cu_count() & ~7;
-  return (int)pick_kv_ds(p)(a, (hipStream_t)stream);
+  a.part = part;
+  a.nparts = nparts;
+  FLEXATT_TRY((int)pick_kv_ds(p)(a, (hipStream_t)stream));
+  if (nparts == 1) return FLEXATT_OK;
+  BwdSplitArgs s;
+  s.dk = a.dk;
+  s.dv = a.dv;
+  s.p = a.p;
+  s.part = part;
+  s.nsplit = nparts;
+  return (int)kPartSum[p->dtype][head_index(p->head_dim)](s, (hipStream_t)stream);
 }
 
 int run_dq_ds(const flexatt_problem* p, const flexatt_tensor* k, const void* workspace, size_t workspace_bytes,
@@ -846,12 +900,19 @@ int flexatt_bwd_dkdv_ds(const flexatt_problem* p, const flexatt_tensor* q, const
                         const flexatt_tensor* v, const flexatt_tensor* dout, const float* lse, const float* delta,
                         const flexatt_tensor* dk, const flexatt_tensor* dv, void* workspace,
                         size_t workspace_bytes, void* stream) {
-  return run_dkdv_ds(p, q, k, v, dout, lse, delta, dk, dv, workspace, workspace_bytes, nullptr, stream);
+  return run_dkdv_ds(p, q, k, v, dout, lse, delta, dk, dv, workspace, workspace_bytes, nullptr, nullptr, 1,
+                     stream);
 }
 
 int flexatt_bwd_dq_ds(const flexatt_problem* p, const flexatt_tensor* k, const void* workspace,
                       size_t workspace_bytes, const flexatt_tensor* dq, void* stream) {
   return run_dq_ds(p, k, workspace, workspace_bytes, dq, nullptr, stream);
+}
+
+size_t flexatt_bwd_ws_parts_bytes(const flexatt_problem* p) {
+  if (check_problem(p) != FLEXATT_OK || !ds_applies(p)) return 0;
+  const int n = staged_parts(p);
+  return n > 1 ? part_bytes(p, n) : 0;
 }
 
 namespace {
@@ -865,7 +926,13 @@ int run_staged(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_
   if (workspace_bytes >= ds_bytes(p) + FLEXATT_BWD_QUEUE_BYTES && (cu_count() & ~7) > 0)
     queue = (int*)((char*)workspace + ds_bytes(p));
   FLEXATT_TRY(run_delta(p, o, dout, delta, queue, stream));
-  FLEXATT_TRY(run_dkdv_ds(p, q, k, v, dout, lse, delta, dk, dv, workspace, workspace_bytes, queue, stream));
+  float* part = nullptr;
+  int nparts = queue ? staged_parts(p) : 1;
+  if (nparts > 1 && workspace_bytes >= ds_bytes(p) + FLEXATT_BWD_QUEUE_BYTES + part_bytes(p, nparts))
+    part = (float*)((char*)workspace + ds_bytes(p) + FLEXATT_BWD_QUEUE_BYTES);
+  else
+    nparts = 1;
+  FLEXATT_TRY(run_dkdv_ds(p, q, k, v, dout, lse, delta, dk, dv, workspace, workspace_bytes, queue, part, nparts, stream));
   return run_dq_ds(p, k, workspace, workspace_bytes, dq, queue ? queue + 2 : nullptr, stream);
 }
 }  // namespace

@@ -43,6 +43,10 @@ struct BwdArgs {
   // otherwise workgroups from nstatic on take their slot from the counter.
   int* queue;
   int nstatic;
+  // Staged dK/dV with each KV block's query tiles shared by nparts workgroups:
+  // their fp32 sums [part][dK, dV][B * Hkv * Skv][D] (nparts == 1: none)
+  float* part;
+  int nparts;
 };
 
 // Split-KV forward (fwd_split.hip): partials in the caller's workspace, none
@@ -121,6 +125,16 @@ hipError_t bwd_split_bf16_d64(const BwdSplitArgs&, hipStream_t);
 hipError_t bwd_split_f16_d64(const BwdSplitArgs&, hipStream_t);
 hipError_t bwd_split_bf16_d128(const BwdSplitArgs&, hipStream_t);
 hipError_t bwd_split_f16_d128(const BwdSplitArgs&, hipStream_t);
+
+// dK and dV from the splits' sums (a.part, a.nsplit), every D.
+hipError_t bwd_split_sum_bf16_d32(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_sum_f16_d32(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_sum_bf16_d64(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_sum_f16_d64(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_sum_bf16_d128(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_sum_f16_d128(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_sum_bf16_d256(const BwdSplitArgs&, hipStream_t);
+hipError_t bwd_split_sum_f16_d256(const BwdSplitArgs&, hipStream_t);
 
 // The same two for fp32 inputs (f32_split.hip; the forward with one split), D <= 128.
 hipError_t fwd_split_f32_d32(const DecodeArgs&, hipStream_t);

@@ -35,6 +35,7 @@ EXPORTS = (
     "flexatt_bwd_prefers_split",
     "flexatt_bwd_split_workspace",
     "flexatt_bwd_split",
+    "flexatt_bwd_ws_parts_bytes",
     "flexatt_bwd_dkdv_ds",
     "flexatt_bwd_dq_ds",
     "flexatt_status_string",
@@ -125,7 +126,7 @@ def load() -> ctypes.CDLL:
         fn.argtypes = args
         fn.restype = ctypes.c_int
     for name in ("flexatt_fwd_decode_workspace", "flexatt_fwd_split_workspace", "flexatt_bwd_workspace",
-                 "flexatt_bwd_split_workspace"):
+                 "flexatt_bwd_split_workspace", "flexatt_bwd_ws_parts_bytes"):
         getattr(lib, name).argtypes = [pr]
         getattr(lib, name).restype = ctypes.c_size_t
     lib.flexatt_bwd_workspace_limited.argtypes = [pr, ctypes.c_size_t]

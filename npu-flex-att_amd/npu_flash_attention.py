@@ -488,6 +488,10 @@ def _backward_into(query, key, value, out, lse, grad_out, DQ, DK, DV, *, causal,
     p = _problem(q, k, scale, causal, sliding_window, soft_cap, slopes, masks)
     split = ds_staging_enabled and ds_staging_auto and lib.flexatt_bwd_prefers_split(p)
     ws_bytes = lib.flexatt_bwd_split_workspace(p) if split else _staged_workspace_bytes(lib, p, query.device)
+    if not split and ws_bytes and ws_bytes == lib.flexatt_bwd_workspace(p):
+        parts = lib.flexatt_bwd_ws_parts_bytes(p)  # whole band: dK/dV may share its blocks' streams
+        if ws_bytes + parts <= _workspace_budget(0):
+            ws_bytes += parts
     with _device_guard(query.device):
         if split:
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device) if ws_bytes else None
