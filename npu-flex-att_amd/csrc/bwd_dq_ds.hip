@@ -43,14 +43,17 @@ namespace flexatt {
 #ifndef FLEXATT_DQ_W256
 #define FLEXATT_DQ_W256 8  // tuning override: 4 waves (one per SIMD, two slots each) at D = 256
 #endif
-template <int D>
+// HALF: two query slots per wave instead of four (D = 64 and 128), so that a
+// grid of few workgroups has twice as many, half as long (launch_dq_ds).
+template <int D, bool HALF>
 struct DqsCfg {
   // waves per workgroup: one per SIMD (D = 64, 128); at D = 256 two per SIMD
   // with one slot each (128 accumulators), so that one wave's loads and LDS
   // reads overlap the other's MFMAs
   static constexpr int NW = D == 256 ? FLEXATT_DQ_W256 : 4;
   static constexpr int WPE = NW / 4;            // waves per SIMD
-  static constexpr int NSL = D == 256 ? 8 / NW : 4;  // query slots per wave (256 accumulators per SIMD at D = 256)
+  // query slots per wave (256 accumulators per SIMD at D = 256)
+  static constexpr int NSL = D == 256 ? 8 / NW : HALF ? 2 : 4;
   static constexpr int SLOTS = NW * NSL;        // query slots per workgroup
   static constexpr int SB = 64;                // KV rows per sub-block
   static constexpr int KS = SB / 16;           // k steps per sub-block
@@ -68,10 +71,11 @@ struct DqsCfg {
   static_assert(KSTAGES * KTILEB <= 128 * 1024, "LDS");
 };
 
-template <class T, int D, bool BLK>
-__global__ __launch_bounds__(DqsCfg<D>::NW * 64) __attribute__((amdgpu_waves_per_eu(DqsCfg<D>::WPE, DqsCfg<D>::WPE)))
+template <class T, int D, bool BLK, bool HALF>
+__global__ __launch_bounds__((DqsCfg<D, HALF>::NW * 64))
+__attribute__((amdgpu_waves_per_eu((DqsCfg<D, HALF>::WPE), (DqsCfg<D, HALF>::WPE))))
 void bwd_dq_ds_kernel(BwdArgs a) {
-  using C = DqsCfg<D>;
+  using C = DqsCfg<D, HALF>;
   using M = Mfma<T>;
   using V8 = typename M::v8;
   static_assert((D == 64 || D == 128 || D == 256) && C::KS == 4, "the MFMA blocking assumes 64-row sub-blocks");
@@ -384,25 +388,42 @@ void bwd_dq_ds_kernel(BwdArgs a) {
   }
 }
 
-template <class T, int D>
-hipError_t launch_dq_ds(const BwdArgs& a, hipStream_t st) {
-  using C = DqsCfg<D>;
+template <class T, int D, bool HALF>
+hipError_t launch_dq_ds(const BwdArgs& a, int nh, int nqb, hipStream_t st) {
+  using C = DqsCfg<D, HALF>;
   BwdArgs x = a;
-  const int nh = (a.p.G % 4 == 0) ? 4 : (a.p.G % 2 == 0) ? 2 : 1;
-  const int nq = C::SLOTS / nh;
-  const int nqt = (a.p.Sq + kDsQT - 1) / kDsQT;
-  const int nqb = (nqt + nq - 1) / nq;
   x.ntiles = (nqb << 8) | nh;
   const dim3 grid(nqb * (a.p.G / nh) * a.p.B * a.p.Hkv), block(C::NW * 64);
   // block-sparse maps: block-map rows of the slots, then the sub-block walk list
   const int nsb = (a.p.Skv + C::SB - 1) / C::SB;
   if (a.p.blk) {
     const size_t dyn = (size_t)C::NW * C::NSL * kBlkRowMax + 2 * (size_t)(nsb + 2);
-    hipLaunchKernelGGL((bwd_dq_ds_kernel<T, D, true>), grid, block, dyn, st, x);
+    hipLaunchKernelGGL((bwd_dq_ds_kernel<T, D, true, HALF>), grid, block, dyn, st, x);
   } else {
-    hipLaunchKernelGGL((bwd_dq_ds_kernel<T, D, false>), grid, block, 0, st, x);
+    hipLaunchKernelGGL((bwd_dq_ds_kernel<T, D, false, HALF>), grid, block, 0, st, x);
   }
   return hipGetLastError();
+}
+
+template <class T, int D>
+hipError_t launch_dq_ds(const BwdArgs& a, hipStream_t st) {
+  const int nh = (a.p.G % 4 == 0) ? 4 : (a.p.G % 2 == 0) ? 2 : 1;
+  const int nqt = (a.p.Sq + kDsQT - 1) / kDsQT;
+  auto blocks = [&](int slots) { return (nqt + slots / nh - 1) / (slots / nh); };
+  const int nqb = blocks(DqsCfg<D, false>::SLOTS);
+  if constexpr (D != 256) {
+    // Workgroups of half the slots where the grid is at most one or two rounds
+    // and they are unequal (causal, masked): the longest one sets the time. Whole
+    // backward, D = 128, us: Hq=32 Hkv=8 S=4096 causal (256 workgroups) 509 -> 479, with
+    // half the blocks masked away 352 -> 315, S=2000 182 -> 149, documents of 700 in
+    // 8192 (512) 584 -> 558.  Equal ones, or two full rounds, keep four: S=4096
+    // non-causal 782 -> 799, B=2 causal (512) 866 -> 871.
+    const int64_t wgs = (int64_t)nqb * (a.p.G / nh) * a.p.B * a.p.Hkv, cus = a.nstatic > 0 ? a.nstatic : 256;
+    const bool masks = a.p.docc || a.p.blk;
+    if (a.p.causal || masks ? wgs < 2 * cus || (masks && wgs == 2 * cus) : 2 * wgs <= cus)
+      return launch_dq_ds<T, D, true>(a, nh, blocks(DqsCfg<D, true>::SLOTS), st);
+  }
+  return launch_dq_ds<T, D, false>(a, nh, nqb, st);
 }
 
 #define FLEXATT_DQ_DS_LAUNCHERS(D)                                                                     \
