@@ -77,3 +77,19 @@ def test_decode_d256_matches_oracle(gpu_device, sq, skv, hq, hkv, cap):
         want, want_lse = orc.forward(*cpu[:3], False, 0, None, 1 / 16, cap)
         check("o", o, want, torch.bfloat16)
         check("lse", lse, want_lse, torch.bfloat16)
+
+
+# (head_dim, partials of a row): 1024 / D partial columns are merged at once, four of each
+@pytest.mark.parametrize("d, ns", [(256, 2), (256, 17), (256, 65), (128, 3), (128, 33), (64, 64), (64, 65), (32, 129),
+                                   (32, 256)])
+def test_merge_of_partials(gpu_device, d, ns):
+    skv = 256 * ns - 5
+    cpu, (q, k, v, _) = draw(ns, 1, 3, 1, 2, skv + 5, d, torch.bfloat16)
+    cpu, (k, v) = (cpu[0], cpu[1][:, :, :skv], cpu[2][:, :, :skv]), (k[:, :, :skv], v[:, :, :skv])
+    p = nfa._problem(q, k, 0.1, False, 0, 0.0, None)
+    # 3 heads x 2 query rows, D + 1 floats a partial
+    assert L.load().flexatt_fwd_split_workspace(p) == 6 * ns * (d + 1) * 4
+    o, lse = nfa.npu_flash_attention_forward(q, k, v, return_lse=True, scale=0.1)
+    want, want_lse = orc.forward(*cpu, False, 0, None, 0.1, 0.0)
+    check("o", o, want, torch.bfloat16)
+    check("lse", lse, want_lse, torch.bfloat16)
