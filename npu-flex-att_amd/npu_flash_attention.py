@@ -176,7 +176,7 @@ def _doc_bounds(document_ids, B, Sq, Sk, device, native=False):
     if ids.dtype.is_floating_point or ids.dtype == torch.bool:
         raise RuntimeError("document_ids must be an integer tensor")
     S = Sk
-    if native and ids.is_cuda and ids.numel() > 0:
+    if native and ids.is_cuda and ids.numel() > 0 and not ids.is_complex():  # (the kernel takes 1 to 8 bytes)
         ids = ids.contiguous()
         bounds = torch.empty(B, S, 2, dtype=torch.int32, device=ids.device)
         with _device_guard(ids.device):

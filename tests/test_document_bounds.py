@@ -30,3 +30,10 @@ def test_bounds_match_tensor_operations(gpu_device, b, s, mean, dtype):
     for x in (ids.cuda(), wide):
         got = nfa._doc_bounds(x, b, s, s, "cuda", native=True)
         assert got.dtype == torch.int32 and torch.equal(got.cpu(), want)
+
+
+@pytest.mark.gpu
+def test_wide_ids_take_tensor_operations(gpu_device):
+    ids = torch.tensor([[1, 1, 2, 2, 2, 1]]).to(torch.complex128)
+    want = nfa._doc_bounds(ids, 1, 6, 6, "cpu")
+    assert torch.equal(nfa._doc_bounds(ids.cuda(), 1, 6, 6, "cuda", native=True).cpu(), want)
