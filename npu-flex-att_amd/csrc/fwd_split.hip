@@ -25,7 +25,9 @@
 //    its LSE in log2 units, in the caller's workspace, and a merge kernel (one
 //    workgroup per row) combines the partials of a row in a fixed
 //    order: M = max LSE_s, O = sum 2^(LSE_s - M) O_s / sum 2^(LSE_s - M),
-//    LSE = (M + log2 sum 2^(LSE_s - M)) ln 2.  Deterministic.
+//    LSE = (M + log2 sum 2^(LSE_s - M)) ln 2.  A partial without keys has LSE
+//    -inf and is left out; one with a NaN score has LSE NaN, which makes the
+//    row's O and LSE NaN.  Deterministic.
 //  * What bounds it: long decodes stream K and V from HBM (two stages per
 //    wave, 5.8 TB/s at bf16 B=8 Hkv=8 Skv=32768 D=128); everything smaller is
 //    a chain of tiles, each one LDS round trip, one softmax and one more round
@@ -310,7 +312,7 @@ void fwd_split_kernel(DecodeArgs a) {
     al[w] = mw[w] == kNegInf ? 0.f : fast_exp2(mw[w] - mall);  // 0 for a wave without keys
     L = __builtin_fmaf(al[w], xl[w * 64 + lane], L);
   }
-  const bool empty = !(L > 0.f);
+  const bool empty = L == 0.f;  // no key; NaN (a NaN query row or key) is not
   const float inv = empty ? 0.f : 1.0f / L;
   if (32 * rt + l32 < R) {
     const int64_t row = ((int64_t)b * p.Hq + hq) * p.Sq + qi;
@@ -356,7 +358,7 @@ __global__ __launch_bounds__(256) void fwd_split_merge_kernel(DecodeArgs a) {
   f32x4 v[U];
   float lw[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {  // (a partial past the last: the last again, at weight 0)
+  for (int u = 0; u < U; ++u) {  // (a partial past the last: the last again, without a weight)
     const int s = g + NG * u, t = min(s, ns - 1);
     v[u] = po[(int64_t)t * TPR];
     lw[u] = s < ns ? pl[t] : kNegInf;
@@ -370,21 +372,22 @@ __global__ __launch_bounds__(256) void fwd_split_merge_kernel(DecodeArgs a) {
   }
 #pragma unroll
   for (int x = 32; x; x >>= 1) mx = fmaxf(mx, __shfl_xor(mx, x));
-  const bool none = mx == kNegInf;  // no allowed key for this row
-  const float m0 = none ? 0.f : mx;
+  const float m0 = mx == kNegInf ? 0.f : mx;
   float ws = 0.f;
 #pragma unroll
   for (int k = 0; k < 4; ++k) ws += fast_exp2(ll[k] - m0);  // 0 for an empty partial
 #pragma unroll
   for (int x = 32; x; x >>= 1) ws += __shfl_xor(ws, x);
+  const bool none = ws == 0.f;  // no allowed key for this row
 
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int s0 = g;;) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const float w = fast_exp2(lw[u] - m0);
+      const bool keys = lw[u] != kNegInf;  // without keys the values do not count, not even an inf
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(w, v[u][j], acc[j]);
+      for (int j = 0; j < 4; ++j) acc[j] = keys ? __builtin_fmaf(w, v[u][j], acc[j]) : acc[j];
     }
     s0 += NG * U;
     if (s0 >= ns) break;

@@ -93,3 +93,20 @@ def test_merge_of_partials(gpu_device, d, ns):
     want, want_lse = orc.forward(*cpu, False, 0, None, 0.1, 0.0)
     check("o", o, want, torch.bfloat16)
     check("lse", lse, want_lse, torch.bfloat16)
+
+
+@pytest.mark.parametrize("what", ["nan_query", "nan_key", "inf_value"])
+@pytest.mark.parametrize("d, sq, skv", [(64, 2, 40), (64, 2, 3000), (128, 2, 3000), (256, 2, 40), (256, 2, 3000),
+                                        (64, 200, 200), (128, 200, 200), (256, 100, 100)])
+def test_nan_and_inf_reach_the_row(gpu_device, d, sq, skv, what):
+    # one workgroup a row tile (40, 100, 200) and partials merged (3000): a row with a NaN score is not an empty row,
+    # and the partials that the merge reads past the last one add nothing
+    cpu, dev = draw(d + skv, 1, 4, 2, sq, skv, d, torch.bfloat16)
+    for q, k, v, _ in (cpu, dev):
+        t, x = {"nan_query": (q[0, 1, 1], "nan"), "nan_key": (k[0, 1, skv - 5], "nan"), "inf_value": (v[0, 0, skv - 5], "inf")}[what]
+        t[3] = float(x)
+    o, lse = nfa.npu_flash_attention_forward(*dev[:3], return_lse=True)
+    want, want_lse = orc.forward(*cpu[:3])
+    assert torch.equal(o.isnan().cpu(), want.isnan()) and torch.equal(lse.isnan().cpu(), want_lse.isnan())
+    check("o", o, want, torch.bfloat16)
+    check("lse", lse, want_lse, torch.bfloat16)
