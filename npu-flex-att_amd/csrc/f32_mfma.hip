@@ -220,7 +220,7 @@ void fwd_f32_kernel(FwdArgs a) {
 
   const float l_tot = l_run + swap_halves(l_run);
   if (my_m < p.Sq) {
-    const bool empty = !(l_tot > 0.f);
+    const bool empty = l_tot == 0.f;  // no key; NaN (a NaN query row or key) is not
     float* op = (float*)a.o.data + b * a.o.sb + hq * a.o.sh + (int64_t)my_m * a.o.ss;
 #pragma unroll
     for (int db = 0; db < C::DB; ++db)

@@ -159,7 +159,7 @@ void fwd_split_f32_kernel(DecodeArgs a) {
     al[v] = mv == kNegInf ? 0.f : expf(mv - m);
     L = fmaf(al[v], xl[v * 64 + lane], L);
   }
-  const bool empty = !(L > 0.f);
+  const bool empty = L == 0.f;  // no key; NaN (a NaN query row or key) is not
   if (32 * rt + l32 < R) {
     float* out = (float*)a.o.data + b * a.o.sb + hq * a.o.sh + (int64_t)qi * a.o.ss + 4 * h;
     for (int x = wave; x < 4 * C::DB; x += kNW) {

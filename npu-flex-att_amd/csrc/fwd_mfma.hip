@@ -601,7 +601,7 @@ void fwd_mfma_kernel(FwdArgs a) {
   }
 
   const float l_tot = l_run + swap_halves(l_run);
-  const bool empty = !(l_tot > 0.f);
+  const bool empty = l_tot == 0.f;  // no key; NaN (a NaN query row or key) is not
   const float inv = empty ? 0.f : 1.0f / l_tot;
   // O leaves through LDS: each lane holds 4 columns of one row, which would
   // make every store instruction touch 32 rows; staged as the wave's 32 x D

@@ -337,7 +337,7 @@ void fwd_ws_kernel(FwdArgs a) {
     }
     // 1 / l to the partner, LSE out
     const float l_tot = l_run + swap_halves(l_run);
-    const bool empty = !(l_tot > 0.f);
+    const bool empty = l_tot == 0.f;  // no key; NaN (a NaN query row or key) is not
     *(float*)(xp(0) + C::XP + lane * 4) = empty ? 0.f : 1.0f / l_tot;
     if (my_m < p.Sq && h == 0)
       a.lse[(int64_t)(b * p.Hq + hq) * p.Sq + my_m] = empty ? kNegInf : (m_run + log2f(l_tot)) * kLn2;

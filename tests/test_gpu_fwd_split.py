@@ -95,18 +95,37 @@ def test_merge_of_partials(gpu_device, d, ns):
     check("lse", lse, want_lse, torch.bfloat16)
 
 
+def _planted(what, d, sq, skv, dtype):
+    cpu, dev = draw(d + skv, 1, 4, 2, sq, skv, d, dtype)
+    for q, k, v, _ in (cpu, dev):
+        t, x = {"nan_query": (q[0, 1, 1], "nan"), "nan_key": (k[0, 1, skv - 5], "nan"), "inf_value": (v[0, 0, skv - 5], "inf")}[what]
+        t[3] = float(x)
+    return cpu, dev
+
+
+def _check_planted(cpu, dev, dtype, **kw):
+    o, lse = nfa.npu_flash_attention_forward(*dev[:3], return_lse=True, **kw)
+    want, want_lse = orc.forward(*cpu[:3])
+    assert torch.equal(o.isnan().cpu(), want.isnan()) and torch.equal(lse.isnan().cpu(), want_lse.isnan())
+    check("o", o, want, dtype)
+    check("lse", lse, want_lse, dtype)
+
+
 @pytest.mark.parametrize("what", ["nan_query", "nan_key", "inf_value"])
 @pytest.mark.parametrize("d, sq, skv", [(64, 2, 40), (64, 2, 3000), (128, 2, 3000), (256, 2, 40), (256, 2, 3000),
                                         (64, 200, 200), (128, 200, 200), (256, 100, 100)])
 def test_nan_and_inf_reach_the_row(gpu_device, d, sq, skv, what):
     # one workgroup a row tile (40, 100, 200) and partials merged (3000): a row with a NaN score is not an empty row,
     # and the partials that the merge reads past the last one add nothing
-    cpu, dev = draw(d + skv, 1, 4, 2, sq, skv, d, torch.bfloat16)
-    for q, k, v, _ in (cpu, dev):
-        t, x = {"nan_query": (q[0, 1, 1], "nan"), "nan_key": (k[0, 1, skv - 5], "nan"), "inf_value": (v[0, 0, skv - 5], "inf")}[what]
-        t[3] = float(x)
-    o, lse = nfa.npu_flash_attention_forward(*dev[:3], return_lse=True)
-    want, want_lse = orc.forward(*cpu[:3])
-    assert torch.equal(o.isnan().cpu(), want.isnan()) and torch.equal(lse.isnan().cpu(), want_lse.isnan())
-    check("o", o, want, torch.bfloat16)
-    check("lse", lse, want_lse, torch.bfloat16)
+    cpu, dev = _planted(what, d, sq, skv, torch.bfloat16)
+    _check_planted(cpu, dev, torch.bfloat16)
+
+
+@pytest.mark.parametrize("what", ["nan_query", "nan_key", "inf_value"])
+@pytest.mark.parametrize("dtype, d", [(torch.bfloat16, 32), (torch.float16, 64), (torch.bfloat16, 128), (torch.bfloat16, 256),
+                                      (torch.float32, 32), (torch.float32, 64), (torch.float32, 128), (torch.float32, 256)])
+def test_nan_and_inf_reach_the_row_in_the_other_kernels(gpu_device, dtype, d, what):
+    # the regular forward (a block map, here of all blocks, keeps a small problem there) and the fp32 kernels
+    cpu, dev = _planted(what, d, 200, 150, dtype)
+    _check_planted(cpu, dev, dtype, block_mask=torch.ones(1, 1, 2, 2, dtype=torch.bool, device="cuda"))
+    _check_planted(cpu, dev, dtype)
