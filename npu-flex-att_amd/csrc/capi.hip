@@ -98,6 +98,13 @@ int check_out_tensor(const flexatt_tensor* t, int dt, int64_t n_b, int64_t n_h, 
   return FLEXATT_OK;
 }
 
+// The window the kernels and the staged-dS layout see, at most Sq: the same mask
+// (i - j < Sq), and neither row + window nor the layout's sums over it leave 32
+// bits, whatever W the caller gives.
+int window_of(const flexatt_problem* p) {
+  return p->sliding_window < p->seqlen_q ? p->sliding_window : p->seqlen_q;
+}
+
 Shape make_shape(const flexatt_problem* p) {
   Shape s;
   s.B = p->batch;
@@ -109,7 +116,7 @@ Shape make_shape(const flexatt_problem* p) {
   s.scale = p->scale;
   s.scale_log2 = p->scale * kLog2e;
   s.causal = p->causal;
-  s.window = p->sliding_window;
+  s.window = window_of(p);
   s.cap = p->soft_cap;
   s.inv_cap = p->soft_cap > 0.f ? 1.0f / p->soft_cap : 0.f;
   s.tanh_k = p->soft_cap > 0.f ? 2.0f * kLog2e * p->scale / p->soft_cap : 0.f;
@@ -196,7 +203,6 @@ int decode_run(const flexatt_problem* p, const DecodePlan& d, const flexatt_tens
   a.o = mview(o);
   a.lse = lse;
   a.p = make_shape(p);
-  if (a.p.window > a.p.Sq) a.p.window = a.p.Sq;  // the same mask
   a.nsplit = d.nsplit;
   a.chunk = d.chunk;
   a.nw = nw;
@@ -409,7 +415,7 @@ BwdLauncher pick_dq_ds(const flexatt_problem* p) {
 int64_t ds_units_per_head(const flexatt_problem* p) {
   const int nqt = (p->seqlen_q + kDsQT - 1) / kDsQT;
   const int nkb = (p->seqlen_kv + kDsKB - 1) / kDsKB;
-  return ds_tile_offset(nqt, p->causal, p->sliding_window, nkb);
+  return ds_tile_offset(nqt, p->causal, window_of(p), nkb);
 }
 size_t ds_bytes(const flexatt_problem* p) {
   if (!ds_applies(p)) return 0;
@@ -814,7 +820,6 @@ int flexatt_bwd_split(const flexatt_problem* p, const flexatt_tensor* q, const f
   a.dk = mview(dk);
   a.dv = mview(dv);
   a.p = c.p;
-  if (a.p.window > a.p.Sq) a.p.window = a.p.Sq;  // the same mask, and no overflow in row + window
   a.part = (float*)workspace;
   a.nsplit = plan.nsplit;
   a.nw = plan.nw;

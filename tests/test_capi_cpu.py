@@ -315,6 +315,20 @@ def test_bwd_workspace_counts_the_band(sq, skv, causal, window):
     assert lib.flexatt_bwd_workspace(p) == 2 * 6 * _staged_units(sq, skv, causal, window) * 8192 + L.BWD_QUEUE_BYTES
 
 
+@pytest.mark.parametrize("sq,skv", [(1, 1), (31, 33), (300, 129), (1000, 257), (129, 1000), (4096, 4096)])
+@pytest.mark.parametrize("dtype", [L.BF16, L.F32])
+@pytest.mark.parametrize("causal", [0, 1])
+def test_any_window_of_at_least_sq_is_no_window(sq, skv, dtype, causal):
+    """i - j < Sq: the staged-dS layout, here its size, is the unwindowed one up to the largest W of the struct (whose
+    sums with a row or a tile would leave 32 bits)."""
+    lib = L.load()
+    kw = dict(batch=2, heads_q=6, heads_kv=2, seqlen_q=sq, seqlen_kv=skv, head_dim=128, causal=causal, dtype=dtype)
+    want = lib.flexatt_bwd_workspace(problem(**kw))
+    for w in (sq, sq + 1, 10 * sq, (1 << 31) - 32, (1 << 31) - 1):
+        assert lib.flexatt_bwd_workspace(problem(sliding_window=w, **kw)) == want
+        assert lib.flexatt_bwd_workspace_limited(problem(sliding_window=w, **kw), 1 << 40) == want
+
+
 def test_bwd_workspace_range():
     lib = L.load()
     ws = lib.flexatt_bwd_workspace

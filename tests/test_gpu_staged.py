@@ -218,6 +218,20 @@ def test_staged_fully_masked_rows(gpu_device, dtype, d):
         check(name, x, r, dtype)
 
 
+@pytest.mark.parametrize("staged", [True, False], ids=["staged", "recomputing"])
+@pytest.mark.parametrize("d", [32, 64, 128, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_widest_window_is_no_window(gpu_device, monkeypatch, dtype, d, staged):
+    """i - j <= W with W >= Sq removes nothing, up to the largest W of the C struct (row + W would leave 32 bits)."""
+    monkeypatch.setattr(nfa, "ds_staging_enabled", staged)
+    cpu, (q, k, v, do) = draw(7, 1, 4, 2, 300, 257, d, dtype)
+    ref = oracle_fwd_bwd(*cpu)
+    for w in (300, (1 << 31) - 1):
+        got = fwd_bwd(nfa, q, k, v, do, sliding_window=w)
+        for name, x, r in zip(("o", "lse", "dq", "dk", "dv"), got, ref):
+            check(name, x, r, dtype)
+
+
 # Grids with more workgroups than CUs: flexatt_bwd_ws hands the workgroups
 # past the first per CU their work items from the queue counters in the
 # workspace (cleared by its Delta pass); the two kernels called on their own
