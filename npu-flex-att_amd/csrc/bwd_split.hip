@@ -8,7 +8,9 @@
 // ALiBi bias, which the reference's backward kernels omit), dP = dO V^T,
 // dS = P (dP - Delta) scale (1 - tanh^2), dV = P^T dO, dK = dS^T Q, dQ = dS K.
 // P and dS are rounded to the input dtype before their MFMAs, as the
-// reference does before tl.dot.
+// reference does before tl.dot: dS with the scale in it at D = 32 and without it
+// above (the gradient is scaled instead), as the other backward kernels of each
+// head dim round it, so that fp16 has one range whatever the size selects.
 //
 // Decomposition
 //  * Two kinds of items in one grid, so that neither waits for the other:
@@ -98,6 +100,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_split_kernel(BwdSplitArgs a) {
   using M = Mfma<T>;
   using V8 = typename M::v8;
   constexpr bool RAW = !SOFTCAP && !ALIBI;
+  constexpr bool SCALED = D == 32;  // dS is rounded with the scale in it
   __shared__ __attribute__((aligned(1024))) char smem[C::LDSB];
 
   const Shape& p = a.p;
@@ -165,6 +168,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_split_kernel(BwdSplitArgs a) {
       float x = fast_exp2(y);
       if (masked) x = (unsigned)(off - lo) < w ? x : 0.f;
       float ds = -x * dp[e];
+      if constexpr (SCALED) ds *= p.scale;
       if constexpr (SOFTCAP) ds *= 1.f - t * t;
       s[e] = x;
       dp[e] = ds;
@@ -269,7 +273,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_split_kernel(BwdSplitArgs a) {
     T* out[2] = {(T*)a.dk.data + b * a.dk.sb + hk * a.dk.sh + (int64_t)row * a.dk.ss + 4 * h,
                  (T*)a.dv.data + b * a.dv.sb + hk * a.dv.sh + (int64_t)row * a.dv.ss + 4 * h};
     combine_waves<2, C::DB, NW>(smem, acc, wave, lane, [&](int i, int db, int qr, f32x4 v) {
-      if (i == 0) v *= p.scale;
+      if (!SCALED && i == 0) v *= p.scale;
       if (!in) return;
       const int col = 32 * db + 8 * qr;
       if (a.nsplit > 1) *(f32x4*)(a.part + (2 * split + i) * pn + prow + col) = v;
@@ -350,7 +354,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_split_kernel(BwdSplitArgs a) {
     const bool in = 32 * rt + l32 < R;
     T* out = (T*)a.dq.data + b * a.dq.sb + hq * a.dq.sh + (int64_t)qi * a.dq.ss + 4 * h;
     combine_waves<1, C::DB, NW>(smem, acc, wave, lane, [&](int, int db, int qr4, f32x4 v) {
-      v *= p.scale;
+      if (!SCALED) v *= p.scale;
       if (in) st_global8(out + 32 * db + 8 * qr4, pack4<T>(v[0], v[1], v[2], v[3]));
     });
   }

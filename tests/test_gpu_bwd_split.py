@@ -94,3 +94,22 @@ def test_other_backward_at_the_same_sizes(gpu_device, monkeypatch, shape, flags)
     o, lse = nfa.npu_flash_attention_forward(q, k, v, return_lse=True, **kw)
     for name, x, r in zip(("dq", "dk", "dv"), nfa.npu_flash_attention_backward(q, k, v, o, lse, do, **kw), want):
         check(name, x, r, dtype)
+
+
+@pytest.mark.parametrize("split", [True, False], ids=["split", "other"])
+@pytest.mark.parametrize("hq, sq", [(2, 8), (6, 8), (2, 33)])
+def test_fp16_d32_rounds_ds_with_the_scale(gpu_device, monkeypatch, hq, sq, split):
+    # large (loss-scaled) gradients: dS reaches 8e4 without the scale, past fp16's 65504, and 1.4e4 with it
+    cpu, dev = draw(3, 1, hq, 2, sq, 5, 32, torch.float16)
+    for q, k, v, do in (cpu, dev):
+        q.mul_(0.1), k.mul_(0.1), v.mul_(2), do.mul_(12000)
+    ds = orc.score_grad(*cpu).abs().max().item()
+    assert 70000 < ds < 65504 * 32 ** 0.5
+    monkeypatch.setattr(nfa, "ds_staging_auto", split)
+    want = orc.backward(*cpu)
+    q, k, v, do = dev
+    p = nfa._problem(q, k, 32 ** -0.5, False, 0, 0.0, None)
+    assert L.load().flexatt_bwd_prefers_split(p) == 1
+    o, lse = nfa.npu_flash_attention_forward(q, k, v, return_lse=True)
+    for name, x, r in zip(("dq", "dk", "dv"), nfa.npu_flash_attention_backward(q, k, v, o, lse, do), want):
+        check(name, x, r, torch.float16)
