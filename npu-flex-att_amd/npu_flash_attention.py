@@ -242,9 +242,12 @@ def _dense_blocks(num, idx, nk, name):
     return out[..., :nk]
 
 
-def _block_map(block_mask, B, Hq, Sq, Sk, device):
+def _block_map(block_mask, B, Hq, Sq, Sk, device, native=False):
     """A block mask in any accepted form -> contiguous uint8 block map
-    [B, Hm, ceil(Sq/128), ceil(Skv/128)] on ``device`` with Hm in {1, Hq}."""
+    [B, Hm, ceil(Sq/128), ceil(Skv/128)] on ``device`` with Hm in {1, Hq}.
+    ``native``: for a call that is over when its kernels are issued; the map
+    may then be the caller's own bool tensor.  A map that is kept (an operator
+    saves it for backward) is always a copy, which the caller may refill."""
     nq, nk = -(-Sq // _BLOCK), -(-Sk // _BLOCK)
     if isinstance(block_mask, torch.Tensor):
         m = block_mask
@@ -253,7 +256,8 @@ def _block_map(block_mask, B, Hq, Sq, Sk, device):
         if m.dim() != 4 or m.shape[2] != nq or m.shape[3] != nk:
             raise RuntimeError(f"a dense block_mask must be [B|1, Hq|1, {nq}, {nk}] (blocks of {_BLOCK}), "
                                f"got {tuple(m.shape)}")
-        m = m.view(torch.uint8) if m.dtype == torch.bool else m != 0  # (a bool is one byte, 0 or 1)
+        # (a bool is one byte, 0 or 1)
+        m = m.view(torch.uint8) if native and m.dtype == torch.bool else m != 0
     else:
         if isinstance(block_mask, (tuple, list)) and len(block_mask) == 2:
             parts = [tuple(block_mask)]
@@ -289,7 +293,7 @@ def _block_map(block_mask, B, Hq, Sq, Sk, device):
 
 def _masks(causal, document_ids, prefix_len, block_mask, B, Hq, Sq, Sk, device, native=False):
     """The interval / block masks of one call as kernel inputs, or None
-    (``native``: see :func:`_doc_bounds`)."""
+    (``native``: see :func:`_doc_bounds` and :func:`_block_map`)."""
     if document_ids is None and block_mask is None and (prefix_len is None or not causal):
         return None
     rows = _doc_bounds(document_ids, B, Sq, Sk, device, native)
@@ -297,7 +301,7 @@ def _masks(causal, document_ids, prefix_len, block_mask, B, Hq, Sq, Sk, device, 
     if prefix_len is not None and causal:
         rows, cols = _prefix_bounds(prefix_len, rows, B, Sq, Sk, device)
         causal = False
-    blocks = _block_map(block_mask, B, Hq, Sq, Sk, device) if block_mask is not None else None
+    blocks = _block_map(block_mask, B, Hq, Sq, Sk, device, native) if block_mask is not None else None
     return _Masks(causal, rows, cols, blocks)
 
 

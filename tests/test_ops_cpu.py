@@ -8,6 +8,7 @@ from torch._subclasses.fake_tensor import FakeTensorMode
 from torch.fx.experimental.proxy_tensor import make_fx
 
 import flexatt_ops
+import npu_flash_attention as nfa
 
 
 def fake_qkv(mode, B=2, Hq=8, Hkv=2, Sq=40, Sk=56, D=64, dtype=torch.bfloat16, grad=False):
@@ -89,3 +90,21 @@ def test_meta_autograd_with_documents():
     o, lse = torch.ops.flexatt.fwd(q, k, v, None, 0.2, True, 0, 0.0, doc)
     o.float().sum().backward()
     assert o.shape == q.shape and k.grad.shape == k.shape
+
+
+def test_block_mask_may_be_refilled_between_forward_and_backward():
+    # the operator saves the map for backward: it is a copy, in bool form too
+    q = torch.empty(2, 8, 140, 64, dtype=torch.bfloat16, device="meta", requires_grad=True)
+    k = torch.empty(2, 2, 56, 64, dtype=torch.bfloat16, device="meta")
+    for dtype in (torch.bool, torch.uint8, torch.int32):
+        mask = torch.ones(2, 8, 2, 1, dtype=dtype, device="meta")
+        o = flexatt_ops.attention(q, k, k, block_mask=mask)
+        mask.fill_(0)
+        o.float().sum().backward()
+
+
+def test_block_map_is_the_callers_tensor_only_in_an_eager_call():
+    mask = torch.tensor([[[[True, False]]]])
+    assert nfa._masks(False, None, None, mask, 1, 1, 128, 256, "cpu").blocks.data_ptr() != mask.data_ptr()
+    m = nfa._masks(False, None, None, mask, 1, 1, 128, 256, "cpu", native=True).blocks
+    assert m.dtype == torch.uint8 and m.tolist() == [[[[1, 0]]]]
