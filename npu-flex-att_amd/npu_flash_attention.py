@@ -472,6 +472,22 @@ def _staged_workspace_bytes(lib, p, device=None) -> int:
     return int(lib.flexatt_bwd_workspace_limited(p, _workspace_budget(free)))
 
 
+def _backward_path(lib, p, device=None):
+    """(split, workspace bytes) of one backward call: flexatt_bwd_split where
+    the library prefers it and the sums it adds fit ``ds_workspace_limit``,
+    else flexatt_bwd_ws, or with 0 bytes flexatt_bwd."""
+    if ds_staging_enabled and ds_staging_auto and lib.flexatt_bwd_prefers_split(p):
+        ws_bytes = int(lib.flexatt_bwd_split_workspace(p))
+        if ws_bytes <= _workspace_budget(0):
+            return True, ws_bytes
+    ws_bytes = _staged_workspace_bytes(lib, p, device)
+    if ws_bytes and ws_bytes == lib.flexatt_bwd_workspace(p):
+        parts = int(lib.flexatt_bwd_ws_parts_bytes(p))  # whole band: dK/dV may share its blocks' streams
+        if ws_bytes + parts <= _workspace_budget(0):
+            ws_bytes += parts
+    return False, ws_bytes
+
+
 def _backward_into(query, key, value, out, lse, grad_out, DQ, DK, DV, *, causal, sliding_window,
                    alibi, scale, soft_cap, masks=None):
     """Run Delta, dQ and dK/dV into the caller's ``DQ`` (kernel-ready layout)
@@ -490,12 +506,7 @@ def _backward_into(query, key, value, out, lse, grad_out, DQ, DK, DV, *, causal,
         lse = lse.to(torch.float32).contiguous()
     slopes = _alibi(alibi, Hq, query.device)
     p = _problem(q, k, scale, causal, sliding_window, soft_cap, slopes, masks)
-    split = ds_staging_enabled and ds_staging_auto and lib.flexatt_bwd_prefers_split(p)
-    ws_bytes = lib.flexatt_bwd_split_workspace(p) if split else _staged_workspace_bytes(lib, p, query.device)
-    if not split and ws_bytes and ws_bytes == lib.flexatt_bwd_workspace(p):
-        parts = lib.flexatt_bwd_ws_parts_bytes(p)  # whole band: dK/dV may share its blocks' streams
-        if ws_bytes + parts <= _workspace_budget(0):
-            ws_bytes += parts
+    split, ws_bytes = _backward_path(lib, p, query.device)
     with _device_guard(query.device):
         if split:
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device) if ws_bytes else None

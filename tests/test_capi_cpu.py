@@ -498,6 +498,36 @@ def test_backward_selects_staging_within_the_limit(monkeypatch):
     assert nfa._staged_workspace_bytes(lib, big) == 0
 
 
+def test_split_and_shared_sums_stay_within_the_limit(monkeypatch):
+    """The workspace budget holds for the split backward's sums and for the shared dK/dV blocks' as for the staged dS."""
+    import npu_flash_attention as nfa
+
+    lib = L.load()
+    p = problem(heads_q=16, heads_kv=1, seqlen_q=640, seqlen_kv=640)
+    n = lib.flexatt_bwd_split_workspace(p)
+    assert lib.flexatt_bwd_prefers_split(p) == 1 and n > 0
+    assert nfa._backward_path(lib, p) == (True, n)
+    monkeypatch.setattr(nfa, "ds_workspace_free_fraction", 0.0)
+    monkeypatch.setattr(nfa, "ds_workspace_limit", n)
+    assert nfa._backward_path(lib, p) == (True, n)
+    for limit in (n - 1, 0):
+        monkeypatch.setattr(nfa, "ds_workspace_limit", limit)
+        assert nfa._backward_path(lib, p) == (False, 0)  # the recomputing backward, which needs none
+    monkeypatch.setattr(nfa, "ds_staging_enabled", False)
+    assert nfa._backward_path(lib, p) == (False, 0)
+    # a split that adds no sums needs no budget
+    monkeypatch.setattr(nfa, "ds_staging_enabled", True)
+    q = problem(heads_q=2, heads_kv=2, seqlen_q=128, seqlen_kv=128)
+    assert lib.flexatt_bwd_split_workspace(q) == 0 and nfa._backward_path(lib, q) == (True, 0)
+    # shared dK/dV blocks: their sums after the whole band, when both fit
+    big = problem(heads_q=32, heads_kv=8, seqlen_q=4096, seqlen_kv=4096, head_dim=128)
+    band, sums = lib.flexatt_bwd_workspace(big), lib.flexatt_bwd_ws_parts_bytes(big)
+    assert sums > 0
+    for limit, want in ((band + sums, band + sums), (band + sums - 1, band), (band, band)):
+        monkeypatch.setattr(nfa, "ds_workspace_limit", limit)
+        assert nfa._backward_path(lib, big) == (False, want)
+
+
 def test_build_rejects_scratch_in_async_load_kernels():
     """The build guard reads the compiler's resource remarks: any kernel of a
     source with asm register loads that uses scratch fails the build."""
