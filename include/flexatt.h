@@ -112,6 +112,11 @@ int flexatt_document_bounds(const void* ids, int ids_bytes, int batch, int seqle
 int flexatt_fwd(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
                 const flexatt_tensor* v, const flexatt_tensor* o, float* lse, void* stream);
 
+/* flexatt_fwd without its choice by size: the kernels of large problems, which
+ * small ones otherwise leave for the split ones (to compare the two). */
+int flexatt_fwd_regular(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
+                        const flexatt_tensor* v, const flexatt_tensor* o, float* lse, void* stream);
+
 /* Split-KV decode forward (flash-decoding): the results of flexatt_fwd for
  * problems with few query rows per KV head, computed by splitting the KV
  * range over many workgroups.  Range: fp16/bf16, head_dim <= 128 and

@@ -495,15 +495,17 @@ const char* flexatt_status_string(int status) {
   }
 }
 
-int flexatt_fwd(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
-                const flexatt_tensor* v, const flexatt_tensor* o, float* lse, void* stream) {
+namespace {
+// `by_size`: the split kernels where split_waves says so, else the regular forward.
+int run_fwd(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k, const flexatt_tensor* v,
+            const flexatt_tensor* o, float* lse, void* stream, bool by_size) {
   FLEXATT_TRY(check_problem(p));
   FLEXATT_TRY(check_tensor(q, p->dtype));
   FLEXATT_TRY(check_tensor(k, p->dtype));
   FLEXATT_TRY(check_tensor(v, p->dtype));
   FLEXATT_TRY(check_out_tensor(o, p->dtype, p->batch, p->heads_q, p->seqlen_q, p->head_dim));
   if (!lse) return FLEXATT_EINVAL;
-  const int nw = split_waves(p);
+  const int nw = by_size ? split_waves(p) : 0;
   if (nw) {
     const DecodePlan d{1, 0, 0, 0};
     return decode_run(p, d, q, k, v, o, lse, nullptr, (hipStream_t)stream, nw);
@@ -517,6 +519,17 @@ int flexatt_fwd(const flexatt_problem* p, const flexatt_tensor* q, const flexatt
   a.p = make_shape(p);
   a.nqt = 0;
   return (int)kFwd[p->dtype][head_index(p->head_dim)](a, (hipStream_t)stream);
+}
+}  // namespace
+
+int flexatt_fwd(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
+                const flexatt_tensor* v, const flexatt_tensor* o, float* lse, void* stream) {
+  return run_fwd(p, q, k, v, o, lse, stream, true);
+}
+
+int flexatt_fwd_regular(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
+                        const flexatt_tensor* v, const flexatt_tensor* o, float* lse, void* stream) {
+  return run_fwd(p, q, k, v, o, lse, stream, false);
 }
 
 size_t flexatt_fwd_decode_workspace(const flexatt_problem* p) {

@@ -18,6 +18,7 @@ F32, F16, BF16 = 0, 1, 2
 EXPORTS = (
     "flexatt_document_bounds",
     "flexatt_fwd",
+    "flexatt_fwd_regular",
     "flexatt_fwd_decode_workspace",
     "flexatt_fwd_decode",
     "flexatt_fwd_split_workspace",
@@ -108,6 +109,7 @@ def load() -> ctypes.CDLL:
     sig = {
         "flexatt_document_bounds": [fp, ctypes.c_int, ctypes.c_int, ctypes.c_int, fp, st],
         "flexatt_fwd": [pr, T, T, T, T, fp, st],
+        "flexatt_fwd_regular": [pr, T, T, T, T, fp, st],
         "flexatt_fwd_decode": [pr, T, T, T, T, fp, fp, ctypes.c_size_t, st],
         "flexatt_fwd_split": [pr, T, T, T, T, fp, fp, ctypes.c_size_t, st],
         "flexatt_fwd_decode_noalloc": [pr, T, T, T, T, fp, st],

@@ -56,8 +56,9 @@ __all__ = [
 _DTYPES = {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 
 # The forward splits the KV range over workgroups (flexatt_fwd_split) whenever
-# the problem is in that range: fp16/bf16 and (Hq / Hkv) * Sq <= 32 (decoding).
-# Set to False to force the regular forward kernel (tests compare the two).
+# the problem is in that range: fp16/bf16 and (Hq / Hkv) * Sq <= 32 (decoding),
+# and otherwise lets flexatt_fwd choose by size.  Set to False to force the
+# regular forward kernel, flexatt_fwd_regular (tests compare the two).
 decode_enabled = True
 # The backward stages dS through a workspace (flexatt_bwd_ws) whenever the
 # library supports it for the problem (fp16/bf16 at head_dim 64, 128 and 256;
@@ -387,8 +388,9 @@ def _forward_into(query, key, value, O, LSE, *, causal, sliding_window, alibi, s
                                        LSE.data_ptr(), ws.data_ptr(), ws_bytes, _stream(query.device))
             _lib.check(st, "flexatt_fwd_split")
             return
-        st = lib.flexatt_fwd(p, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v), _lib.tensor(O),
-                             LSE.data_ptr(), _stream(query.device))
+        fwd = lib.flexatt_fwd if decode_enabled else lib.flexatt_fwd_regular
+        st = fwd(p, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v), _lib.tensor(O), LSE.data_ptr(),
+                 _stream(query.device))
     _lib.check(st, "flexatt_fwd")
 
 
