@@ -328,6 +328,15 @@ int64_t attended_pairs(const flexatt_problem* p) {
 // S=4096 non-causal 1126 -> 753; D = 64 H=2 S=2048 318 -> 55; D = 32 H=8 S=2048 204
 // -> 43.  The estimate of a full chip (5.9 us per 1024 pairs at D = 128, the
 // regular kernel 4.5) keeps large problems on the regular kernel.
+// Many row tiles of few keys: each 32-row workgroup costs its launch, its Q rows
+// and its combine, `wg` us per 1024 of them besides `pair` per 1024 tile pairs,
+// which the regular kernel's one chain (0.6 us a tile, and 2 us more around it) must
+// outlast.  Fitted to 1700 shapes, 33 .. 5000 positions, B = 1 .. 8, windowed, causal
+// and not; without this term 5% of them were slower than the regular kernel: bf16
+// D = 128 B=8 Hq=32 Hkv=8 S=143 causal 11.9 (regular) against 18.0, window 32 Hq=32 Hkv=8
+// Sq=2286 Skv=72 16.0 against 23.4; D = 64 B=4 Hq=128 Hkv=16 S=144 causal 11.4 against 15.3;
+// fp32 D = 128 B=4 Hq=56 Hkv=8 S=183 73 against 108; with it none of 1300 others by 8%, and 97% of
+// the gain stays.  D = 256 loses its 1 us at one or two tiles of keys (S=42 8.7 against 10.1).
 int split_waves(const flexatt_problem* p) {
   if (p->block_map || !kSplit[p->dtype][head_index(p->head_dim)]) return 0;
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
@@ -341,15 +350,18 @@ int split_waves(const flexatt_problem* p) {
   const int64_t chain = (keys + 31) / 32;
   const int64_t units = groups * G * attended_pairs(p) / (32 * 32);
   if (p->dtype == FLEXATT_F32) {
-    constexpr double tile[3] = {1.9, 3.2, 5.85}, unit[3] = {1.7, 2.9, 5.9}, other[3] = {3.2, 5.0, 8.4};
+    constexpr double tile[3] = {1.9, 3.2, 5.85}, unit[3] = {1.7, 2.9, 5.9}, other[3] = {3.2, 5.0, 8.4}, wg[3] = {5, 15, 32};
     const int d = head_index(p->head_dim);
-    const double c = tile[d] * chain / 4, w = unit[d] * units / 1024;
-    return 5 + (c > w ? c : w) < 6 + other[d] * chain ? 4 : 0;
+    const double c = tile[d] * chain / 4, w = (unit[d] * units + wg[d] * wgs) / 1024;
+    const double rows = p->seqlen_q <= 128 ? 0.6 : 1.0;  // the regular workgroup then runs one wave a SIMD
+    return 5 + (c > w ? c : w) < 6 + rows * other[d] * chain ? 4 : 0;
   }
-  if (p->head_dim == 256) return wgs <= cus ? 4 : 0;
+  if (p->head_dim == 256) return wgs <= cus && chain > 2 ? 4 : 0;
   // (an eighth above the measured points, whose causal pairs are just over half)
   const int64_t load = 8 * units / (cus * chain);  // in eighths
   if (load > (p->head_dim == 128 ? 18 : 36)) return 0;
+  constexpr double pair[3] = {0.3, 0.5, 0.85}, wg[3] = {2.5, 3.7, 9.2};
+  if ((pair[head_index(p->head_dim)] * units + wg[head_index(p->head_dim)] * wgs) / 1024 > 2 + 0.6 * chain) return 0;
   if (p->head_dim == 128) return wgs <= cus && chain >= 64 && load <= 9 ? 8 : 4;
   return wgs <= cus && chain >= 32 ? 8 : 4;
 }
