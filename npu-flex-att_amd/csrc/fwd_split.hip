@@ -80,10 +80,14 @@ void fwd_split_kernel(DecodeArgs a) {
 
   // Work item: (b, hkv, row tile, split); the splits of one row tile are
   // consecutive, and its last row tile (the longest causal range) goes first.
+  // Row tiles of one (b, hkv) share an XCD; a single one (decoding) has nothing
+  // to share, and contiguous ranges per XCD then only bunch the cache's
+  // addresses: bf16 D=64 B=128 Hq=32 Hkv=8 Skv=8192 389 -> 367 us in plain order,
+  // D=32 Skv=16384 384 -> 370, D=128 B=64 704 -> 700.
   const int s = blockIdx.x % a.nsplit;
   const int item = blockIdx.x / a.nsplit;
   int krt, bh;
-  if (a.nsplit > 1 || !xcd_lpt_item(item, a.nrt, p.B * p.Hkv, krt, bh)) {
+  if (a.nsplit > 1 || a.nrt == 1 || !xcd_lpt_item(item, a.nrt, p.B * p.Hkv, krt, bh)) {
     krt = item % a.nrt;
     bh = item / a.nrt;
   }
@@ -435,6 +439,8 @@ hipError_t launch_split(const DecodeArgs& a, hipStream_t st) {
   if constexpr (D == 256) {
     return launch_split<T, D, 4, 1>(x, st);
   } else {
+    // (one split of a long cache, a batch with a workgroup or more per slot: ST = 1
+    // and 2 within 2% at 8192 and 16384 keys, ST = 1 ahead at 500, D = 128 42 against 48 us)
     if (x.nsplit > 1) return launch_split<T, D, 4, 2>(x, st);
     if (x.nw == 8) return launch_split<T, D, 8, 1>(x, st);
     return launch_split<T, D, 4, 1>(x, st);

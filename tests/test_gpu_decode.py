@@ -13,6 +13,7 @@ import torch
 import flexatt_lib as L
 import npu_flash_attention as nfa
 from gpu_helpers import alibi_slopes, check, draw, oracle_fwd_bwd
+from oracle import attention_oracle as orc
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +89,16 @@ def test_backward_after_decode_forward(gpu_device):
     ref = oracle_fwd_bwd(*cpu, **kw)
     for name, x, r in zip(("dq", "dk", "dv"), (dq, dk, dv), ref[2:]):
         check(name, x, r, dtype)
+
+
+@pytest.mark.parametrize("d, b, hq, hkv, sq, skv", [(32, 520, 1, 1, 1, 70), (64, 90, 12, 6, 3, 300), (128, 130, 8, 4, 2, 333),
+                                                    (256, 65, 8, 8, 1, 290)])
+def test_large_batches_take_one_split(gpu_device, d, b, hq, hkv, sq, skv):
+    # 512 (batch, KV head) pairs or more: one workgroup each, which writes O and LSE itself
+    cpu, (q, k, v, _) = draw(d, b, hq, hkv, sq, skv, d, torch.bfloat16)
+    n = L.load().flexatt_fwd_split_workspace(nfa._problem(q, k, d ** -0.5, False, 0, 0.0, None))
+    assert n == b * hq * sq * (d + 1) * 4  # of one split
+    o, lse = nfa.npu_flash_attention_forward(q, k, v, return_lse=True)
+    want, want_lse = orc.forward(*cpu[:3])
+    check("o", o, want, torch.bfloat16)
+    check("lse", lse, want_lse, torch.bfloat16)
