@@ -697,31 +697,54 @@ int flexatt_bwd(const flexatt_problem* p, const flexatt_tensor* q, const flexatt
 }
 
 namespace {
-// Workgroups that share the query tiles of one KV block in the staged dK/dV
-// launch (fp16/bf16).  With one item per KV block and no more items than CUs the
-// launch lasts as long as its longest block, and under a causal mask the
-// average one is half as long: about two items per CU even that out
-// (longest first).  More cost their fp32 sums.  Backward, parts 1 / 2 / 3 / 4, us, D = 128
-// causal: Hq=32 Hkv=8 S=4096 604 / 501 / 515 / 523 (256 blocks), with half the blocks
-// masked away 477 / 345 / 351 / 362, S=3000 429 / 333 / 318 / 331 (192), S=2048 295 / 218 /
-// 194 / 194 (128), Hkv=16 S=4096 479 / 532 (512); non-causal, whose blocks are equally long
-// and fill one round: S=2048 300 / 246 / 282 / 265, S=4096 785 / 835; D = 64, two workgroups a
-// CU: half the blocks masked S=4096 416 / 311 / 285 / 272; D = 256, two passes a block:
-// Hq=16 S=1000 141 / 102 / 97 / 101, S=4096 565 / 582.
-int staged_parts(const flexatt_problem* p) {
-  if (!is_16bit(p) || p->head_dim == 32) return 1;
-  const int cus = cu_count() > 0 ? cu_count() : 256;
-  const int64_t items = (int64_t)p->batch * p->heads_kv * ((p->seqlen_kv + kDsKB - 1) / kDsKB) * (p->head_dim == 256 ? 2 : 1);
-  const int64_t slots = p->head_dim == 64 ? 2 * cus : cus;
-  // blocks equally long: no causal mask, or a window that most of them see whole
-  const bool uniform = !has_masks(p) && (!p->causal || (p->sliding_window > 0 && p->sliding_window <= p->seqlen_q / 4));
-  int64_t n = uniform ? slots / items : (2 * slots + items / 2) / items;
-  const int64_t most = (p->seqlen_q + 4 * kDsQT - 1) / (4 * kDsQT);  // at least about four query tiles each
-  if (n > most) n = most;
-  return (int)(n > 4 ? 4 : n < 1 ? 1 : n);
-}
 size_t part_bytes(const flexatt_problem* p, int nparts) {
   return 2 * sizeof(float) * (size_t)nparts * p->batch * p->heads_kv * p->seqlen_kv * p->head_dim;
+}
+// Interval and block masks are device data: the longest walk and the work that
+// the host counts for a problem, times this and its square, are what packed documents of
+// 40 .. 8000 positions measured closest to (either way from 0.6 to 0.8).
+double mask_share(const flexatt_problem* p) { return has_masks(p) ? 0.7 : 1.0; }
+
+// Workgroups that share the query tiles of one KV block in the staged dK/dV
+// launch (fp16/bf16).  The launch lasts as long as its longest block, or as the
+// work per CU where that is longer; parts divide the first and cost their fp32 sums,
+// written and read at about 5.5 TB/s, and their launch.  Estimates in us, fitted to
+// 940 shapes (450 without documents: H = 1 .. 128, G = 1 .. 8, 64 .. 8000 positions, causal,
+// windowed and not; 490 with them): `tile` per 32-row query tile of the longest block, `work`
+// per tile and CU, `start` per 1024 workgroups.  Of those shapes 10 without and 28 with
+// documents are more than 5% slower than one part; a rule that counted blocks
+// against CUs had 44 and 77.  Backward, parts 1 / 2 / 3 / 4, us, D = 128 causal: Hq=32
+// Hkv=8 S=4096 604 / 501 / 515 / 523, S=3000 429 / 333 / 318 / 331, S=2048 295 / 218 / 194 /
+// 194; documents of 100 on average S=3000 90 / 98 / 111, of 2000 310 / - / 226; Hq=Hkv=16 S=2048 of
+// 200 53 / 76 (G = 1: short walks, the same sums); D = 64 with half the blocks masked S=4096 416 / 311 / 285 /
+// 272; D = 256 Hq=16 S=1000 141 / 102 / 97 / 101.
+int staged_parts(const flexatt_problem* p) {
+  if (!is_16bit(p) || p->head_dim == 32) return 1;
+  const int d = head_index(p->head_dim);
+  constexpr double tile[4] = {0, 0.91, 0.78, 0.94}, work[4] = {0, 0.92, 1.08, 1.0}, start[4] = {0, 0, 5.5, 5.0};
+  const double cus = cu_count() > 0 ? cu_count() : 256, slots = p->head_dim == 64 ? 2 * cus : cus;
+  const int passes = p->head_dim == 256 ? 2 : 1;
+  const int64_t nkb = (p->seqlen_kv + kDsKB - 1) / kDsKB, blocks = (int64_t)p->batch * p->heads_kv * nkb * passes;
+  int64_t walk = (p->seqlen_q + kDsQT - 1) / kDsQT;  // query tiles of the longest block
+  if (p->sliding_window > 0) {
+    const int64_t w = ((p->causal ? kDsKB : nkb * kDsKB) + window_of(p) + kDsQT - 1) / kDsQT;
+    if (w < walk) walk = w;
+  }
+  const double share = mask_share(p), cap = p->soft_cap > 0.f ? 1.2 : 1.0;
+  const double longest = tile[d] * cap * share * walk * (p->heads_q / p->heads_kv);
+  const double even = work[d] * cap * share * share * passes * p->batch * p->heads_q * ds_units_per_head(p) / slots;
+  const int64_t most = (p->seqlen_q + 4 * kDsQT - 1) / (4 * kDsQT);  // at least about four query tiles each
+  double best = 1e30;
+  int parts = 1;
+  for (int n = 1; n <= 4 && n <= most; ++n) {
+    const double busy = even + start[d] * n * blocks / 1024, one = longest / n;
+    const double est = (one > busy ? one : busy) + (n > 1 ? 0.7 + 0.01 * longest + 0.36e-6 * part_bytes(p, n) : 0.0);
+    if (est < best) {
+      best = est;
+      parts = n;
+    }
+  }
+  return parts;
 }
 
 const BwdSplitLauncher kBwdSplit[3][4] = {
