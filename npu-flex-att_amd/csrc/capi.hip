@@ -711,7 +711,7 @@ double mask_share(const flexatt_problem* p) { return has_masks(p) ? 0.7 : 1.0; }
 // written and read at about 5.5 TB/s, and their launch.  Estimates in us, fitted to
 // 940 shapes (450 without documents: H = 1 .. 128, G = 1 .. 8, 64 .. 8000 positions, causal,
 // windowed and not; 490 with them): `tile` per 32-row query tile of the longest block, `work`
-// per tile and CU, `start` per 1024 workgroups.  Of those shapes 10 without and 28 with
+// per tile and CU, `start` per 1024 workgroups, `sums` for their launch.  Of those shapes 7 without and 27 with
 // documents are more than 5% slower than one part; a rule that counted blocks
 // against CUs had 44 and 77.  Backward, parts 1 / 2 / 3 / 4, us, D = 128 causal: Hq=32
 // Hkv=8 S=4096 604 / 501 / 515 / 523, S=3000 429 / 333 / 318 / 331, S=2048 295 / 218 / 194 /
@@ -721,7 +721,7 @@ double mask_share(const flexatt_problem* p) { return has_masks(p) ? 0.7 : 1.0; }
 int staged_parts(const flexatt_problem* p) {
   if (!is_16bit(p) || p->head_dim == 32) return 1;
   const int d = head_index(p->head_dim);
-  constexpr double tile[4] = {0, 0.91, 0.78, 0.94}, work[4] = {0, 0.92, 1.08, 1.0}, start[4] = {0, 0, 5.5, 5.0};
+  constexpr double tile[4] = {0, 0.91, 0.78, 0.94}, work[4] = {0, 0.92, 1.08, 1.0}, start[4] = {0, 0, 5.5, 5.0}, sums[4] = {0, 2.5, 0.7, 2.5};
   const double cus = cu_count() > 0 ? cu_count() : 256, slots = p->head_dim == 64 ? 2 * cus : cus;
   const int passes = p->head_dim == 256 ? 2 : 1;
   const int64_t nkb = (p->seqlen_kv + kDsKB - 1) / kDsKB, blocks = (int64_t)p->batch * p->heads_kv * nkb * passes;
@@ -738,7 +738,7 @@ int staged_parts(const flexatt_problem* p) {
   int parts = 1;
   for (int n = 1; n <= 4 && n <= most; ++n) {
     const double busy = even + start[d] * n * blocks / 1024, one = longest / n;
-    const double est = (one > busy ? one : busy) + (n > 1 ? 0.7 + 0.01 * longest + 0.36e-6 * part_bytes(p, n) : 0.0);
+    const double est = (one > busy ? one : busy) + (n > 1 ? sums[d] + 0.01 * longest + 0.36e-6 * part_bytes(p, n) : 0.0);
     if (est < best) {
       best = est;
       parts = n;
