@@ -705,6 +705,15 @@ size_t part_bytes(const flexatt_problem* p, int nparts) {
 // 40 .. 8000 positions measured closest to (either way from 0.6 to 0.8).
 double mask_share(const flexatt_problem* p) { return has_masks(p) ? 0.7 : 1.0; }
 
+// 32-row query tiles that the longest KV block of the staged dK/dV walks for one head.
+int64_t longest_walk(const flexatt_problem* p) {
+  const int64_t nqt = (p->seqlen_q + kDsQT - 1) / kDsQT;
+  if (p->sliding_window == 0) return nqt;
+  const int64_t keys = p->causal ? kDsKB : (p->seqlen_kv + kDsKB - 1) / kDsKB * (int64_t)kDsKB;
+  const int64_t w = (keys + window_of(p) + kDsQT - 1) / kDsQT;
+  return w < nqt ? w : nqt;
+}
+
 // Workgroups that share the query tiles of one KV block in the staged dK/dV
 // launch (fp16/bf16).  The launch lasts as long as its longest block, or as the
 // work per CU where that is longer; parts divide the first and cost their fp32 sums,
@@ -721,17 +730,13 @@ double mask_share(const flexatt_problem* p) { return has_masks(p) ? 0.7 : 1.0; }
 int staged_parts(const flexatt_problem* p) {
   if (!is_16bit(p) || p->head_dim == 32) return 1;
   const int d = head_index(p->head_dim);
-  constexpr double tile[4] = {0, 0.91, 0.78, 0.94}, work[4] = {0, 0.92, 1.08, 1.0}, start[4] = {0, 0, 5.5, 5.0}, sums[4] = {0, 2.5, 0.7, 2.5};
+  constexpr double tile[4] = {0, 0.91, 0.78, 0.94}, work[4] = {0, 0.92, 1.08, 1.0};
+  constexpr double start[4] = {0, 0, 5.5, 5.0}, sums[4] = {0, 2.5, 0.7, 2.5};
   const double cus = cu_count() > 0 ? cu_count() : 256, slots = p->head_dim == 64 ? 2 * cus : cus;
   const int passes = p->head_dim == 256 ? 2 : 1;
   const int64_t nkb = (p->seqlen_kv + kDsKB - 1) / kDsKB, blocks = (int64_t)p->batch * p->heads_kv * nkb * passes;
-  int64_t walk = (p->seqlen_q + kDsQT - 1) / kDsQT;  // query tiles of the longest block
-  if (p->sliding_window > 0) {
-    const int64_t w = ((p->causal ? kDsKB : nkb * kDsKB) + window_of(p) + kDsQT - 1) / kDsQT;
-    if (w < walk) walk = w;
-  }
   const double share = mask_share(p), cap = p->soft_cap > 0.f ? 1.2 : 1.0;
-  const double longest = tile[d] * cap * share * walk * (p->heads_q / p->heads_kv);
+  const double longest = tile[d] * cap * share * longest_walk(p) * (p->heads_q / p->heads_kv);
   const double even = work[d] * cap * share * share * passes * p->batch * p->heads_q * ds_units_per_head(p) / slots;
   const int64_t most = (p->seqlen_q + 4 * kDsQT - 1) / (4 * kDsQT);  // at least about four query tiles each
   double best = 1e30;
@@ -756,42 +761,57 @@ bool bwd_split_applies(const flexatt_problem* p) {
   return kBwdSplit[p->dtype][head_index(p->head_dim)] && !p->block_map;
 }
 // The split backward's plan, and whether it beats the staged / recomputing
-// backward, from estimates in us fitted to graph replays of 56 bf16 shapes
-// (H = 2 .. 32, G = 1 and 4, S = 128 .. 2048, B = 1 .. 4, causal, windowed and not).
-// A workgroup's time is its longest chain of 32 x 32 tiles (D = 128: 1.6 us a tile
-// and wave; 64: 1.2, 1.4 with eight waves, two to a SIMD; 32: 0.8) until the chip is full;
+// backward, from estimates in us fitted to graph replays of 950 shapes without documents
+// (H = 1 .. 128, G = 1 .. 8, 64 .. 8000 positions, B = 1 .. 8, causal, windowed and not).
+// A workgroup's time is its longest chain of 32 x 32 tiles (D = 128: 1.9 us a tile
+// and wave; 64: 1.45, 1.7 with eight waves, two to a SIMD; 32: 0.8) until the chip is full;
 // then the chip's time is `unit` per 1024 tile pairs and `wg` per 1024
-// workgroups.  The other backward's time, until its own grid fills the chip, is
-// its longest dK/dV chain (G heads of the query tiles) and its longest dQ chain.
+// workgroups.  The other backward's (BwdOtherCost) is its longest dK/dV walk, divided by
+// staged_parts, or the work per CU, and its longest dQ chain or the work; interval masks
+// count for mask_share.  Taken at 10% less.  Of 1550 shapes that neither this nor staged_parts was
+// fitted to, 19 are more than 5% slower than the other backward without parts, the worst 1.4
+// times; constants fitted to 56 shapes, without the work on the other side, had 106.
 // Measured, other -> split (waves x splits): D = 64 H=2 S=2048 causal 75 -> 20
 // (8 x 1), Hq=8 Hkv=2 S=2048 193 -> 41 (8 x 2); D = 128 Hq=8 Hkv=2 S=1000 155
-// -> 34 (4 x 4), S=2048 286 -> 74 (4 x 2), Hq=32 Hkv=8 S=2048 295 -> 242 (4 x 1); past
-// the crossover: Hq=32 Hkv=8 B=2 S=2048 D=128 326 -> 472, D=64 242 -> 217 (not taken).
+// -> 34 (4 x 4), S=2048 286 -> 74 (4 x 2); past the crossover: Hq=32 Hkv=8 B=2 S=2048 D=128
+// 326 -> 472; D = 128 B=4 H=4 S=1099 73 -> 92, B=8 Hq=8 Hkv=8 S=347 causal 39 -> 51; D = 64 B=4
+// Hq=64 Hkv=8 S=1522 documents of 1000 on average 425 -> 533.
 struct BwdSplitPlan {
   bool faster;
   int nsplit, nw;
   size_t bytes;
 };
-// fp32 (four waves; 30 shapes): D = 128 10 us a tile and wave, 19.5 us per 1024
-// pairs (the other backward 11 once it fills the chip, which its estimate, a
-// chain, does not count, so that large problems stay with it).  Other -> split:
-// Hq=8 Hkv=2 S=1000 D=128 1264 -> 108 (4 x 4), H=2 S=2048 D=64 480 -> 93 (4 x 1).
+// fp32 (four waves; 250 of the shapes): D = 128 10 us a tile and wave, 19.5 us per 1024
+// pairs.  Other -> split: Hq=8 Hkv=2 S=1000 D=128 1264 -> 108 (4 x 4), H=2 S=2048 D=64 480
+// -> 93 (4 x 1); past the crossover: D = 128 B=8 H=2 Sq=107 Skv=7443 causal 71 -> 112.
 struct BwdSplitCost {
-  double tile4, tile8, base4, base8, unit, wg4, wg8, other, other_kv, other_q;
+  double tile4, tile8, base4, base8, unit, wg4, wg8;
 };
 constexpr BwdSplitCost kBwdSplitCost[2][3] = {
-    {{0.8, 1.0, 6.0, 7.0, 1.0, 5.0, 10.0, 16.0, 0.65, 0.6},    // fp16/bf16, D = 32
-     {1.2, 1.4, 7.0, 8.5, 1.4, 8.0, 14.0, 14.0, 0.62, 0.4},    // 64
-     {1.6, 0.0, 9.0, 0.0, 2.8, 20.0, 0.0, 20.0, 0.95, 0.9}},   // 128 (four waves only)
-    {{3.5, 0.0, 7.0, 0.0, 5.5, 8.0, 0.0, 10.0, 3.3, 1.2},      // fp32, D = 32
-     {5.7, 0.0, 8.0, 0.0, 9.0, 8.0, 0.0, 10.0, 5.3, 1.9},      // 64
-     {10.0, 0.0, 10.0, 0.0, 19.5, 10.0, 0.0, 10.0, 9.2, 4.0}}, // 128
+    {{0.8, 1.0, 6.0, 7.0, 1.0, 5.0, 10.0},     // fp16/bf16, D = 32
+     {1.45, 1.7, 7.5, 8.0, 1.5, 9.0, 16.0},    // 64
+     {1.9, 0.0, 9.5, 0.0, 3.0, 22.0, 0.0}},    // 128 (four waves only)
+    {{3.5, 0.0, 7.0, 0.0, 5.5, 8.0, 0.0},      // fp32, D = 32
+     {5.7, 0.0, 8.0, 0.0, 9.0, 8.0, 0.0},      // 64
+     {10.3, 0.0, 13.0, 0.0, 19.5, 44.0, 0.0}}, // 128
 };
+// The other backward: us around its kernels, per 32-row query tile of the longest dK/dV walk and per tile and CU of all,
+// per 32-key tile of the longest dQ chain and per 1024 tile pairs (0: the chain alone decided the fit).
+struct BwdOtherCost {
+  double base, kv, kv_work, q, q_work;
+};
+BwdOtherCost bwd_other_cost(const flexatt_problem* p, bool staged) {
+  const int d = head_index(p->head_dim);
+  constexpr BwdOtherCost f32[3] = {{10.0, 3.3, 0.0, 1.2, 0.0}, {10.0, 5.3, 0.0, 1.9, 0.0}, {6.8, 8.1, 0.0, 5.1, 8.35}};
+  constexpr BwdOtherCost half[3] = {{16.0, 0.65, 0.0, 0.6, 0.0}, {15.2, 0.69, 1.52, 0.33, 0.53}, {20.7, 0.94, 1.12, 0.46, 0.79}};
+  constexpr BwdOtherCost half64_staged = {17.0, 1.11, 1.4, 0.15, 1.06};
+  return p->dtype == FLEXATT_F32 ? f32[d] : d == 1 && staged ? half64_staged : half[d];
+}
 BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
   const bool f32 = p->dtype == FLEXATT_F32;
   const BwdSplitCost& c = kBwdSplitCost[f32][head_index(p->head_dim)];
   const bool cap = p->soft_cap > 0.f;
-  const double G = p->heads_q / p->heads_kv, groups = (double)p->batch * p->heads_kv;
+  const double G = p->heads_q / p->heads_kv, groups = (double)p->batch * p->heads_kv, share = mask_share(p);
   const int64_t nqt = (p->seqlen_q + 31) / 32, nkt = (p->seqlen_kv + 31) / 32;
   int64_t lq = nqt, lk = nkt;  // longest streams: query tiles of a KV item, key tiles of a Q item
   if (p->causal && nqt < lk) lk = nqt;
@@ -800,7 +820,7 @@ BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
     if (l < lq) lq = l;
     if (l < lk) lk = l;
   }
-  const double units = groups * G * (double)attended_pairs(p) / (32.0 * 32 * 1024);
+  const double units = share * share * groups * G * (double)attended_pairs(p) / (32.0 * 32 * 1024);
   const int64_t nrt = ((int64_t)(p->heads_q / p->heads_kv) * p->seqlen_q + 31) / 32;
   const double part = 2.0 * sizeof(float) * groups * p->seqlen_kv * p->head_dim;  // bytes of one split's sums
   double best = 1e30;
@@ -809,10 +829,10 @@ BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
     for (int ns = 1; ns <= 8; ns *= 2) {
       const double t = nw == 8 ? c.tile8 : c.tile4, base = nw == 8 ? c.base8 : c.base4;
       const double wgs = groups * (double)(nkt * ns + nrt) / 1024;
-      const double chain = t * (G * lq / ns > lk ? G * lq / ns : lk) / nw;
+      const double chain = t * share * (G * lq / ns > lk ? G * lq / ns : lk) / nw;
       const double work = c.unit * (cap ? 1.25 : 1.0) * units + (nw == 8 ? c.wg8 : c.wg4) * wgs;
-      // the sums written and read back at about 8 TB/s (they stay in cache), and one more launch
-      const double est = base + (chain > work ? chain : work) + (ns > 1 ? 4 + 2 * ns * part / 8e6 : 0);
+      // the sums written and read back at about 7 TB/s (they stay in cache), and one more launch
+      const double est = base + (chain > work ? chain : work) + (ns > 1 ? 4 + 0.3e-6 * ns * part : 0);
       if (est < best) {
         best = est;
         r.nsplit = ns;
@@ -820,14 +840,16 @@ BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
       }
     }
   // the staged backward where it is preferred, its dK/dV streams shared by parts
-  const int np = flexatt_bwd_prefers_staging(p) ? staged_parts(p) : 1;
-  double other = c.other + c.other_kv * (cap ? 1.2 : 1.0) * G * lq / np + c.other_q * lk;
-  if (p->head_dim == 64 && cap && !f32) other = 20 + 1.22 * G * lq / np + c.other_q * lk;
-  if (np > 1) {
-    const double work = 25 + 1.75 * units;
-    other = (other > work ? other : work) + 8 + 2 * np * part / 8e6;
-  }
-  r.faster = best < other;
+  const bool staged = flexatt_bwd_prefers_staging(p);
+  const int np = staged ? staged_parts(p) : 1;
+  const BwdOtherCost o = bwd_other_cost(p, staged);
+  const double cus = cu_count() > 0 ? cu_count() : 256, slots = p->head_dim == 64 ? 2 * cus : cus;
+  const double walk = o.kv * share * G * longest_walk(p) / np;
+  const double even = o.kv_work * share * share * p->batch * p->heads_q * ds_units_per_head(p) / slots;
+  const double dq = o.q * share * lk, dq_even = o.q_work * units;
+  const double other = o.base + (cap ? 1.2 : 1.0) * (walk > even ? walk : even) + (dq > dq_even ? dq : dq_even) +
+                       (np > 1 ? 3 + 0.38e-6 * np * part : 0.0);
+  r.faster = best < 0.9 * other;
   if (r.nsplit > 1) r.bytes = (size_t)(part * r.nsplit);
   return r;
 }

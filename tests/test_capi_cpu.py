@@ -548,6 +548,24 @@ def test_kv_blocks_are_shared_where_it_pays(kw, parts):
     assert L.load().flexatt_bwd_ws_parts_bytes(p) == (parts * one if parts > 1 else 0)
 
 
+@pytest.mark.parametrize("kw, split", [
+    (dict(heads_q=2, heads_kv=2, seqlen_q=2048, seqlen_kv=2048), 1),
+    (dict(heads_q=8, heads_kv=2, seqlen_q=1000, seqlen_kv=1000, head_dim=128), 1),
+    (dict(heads_q=8, heads_kv=2, seqlen_q=1000, seqlen_kv=1000, head_dim=128, dtype=L.F32), 1),
+    (dict(batch=4, heads_q=8, heads_kv=8, seqlen_q=1021, seqlen_kv=1021, head_dim=32, sliding_window=256), 1),
+    (dict(heads_q=32, heads_kv=8, seqlen_q=1000, seqlen_kv=1000, doc_bounds=FAKE), 1),
+    # the other backward measured 1.1 to 1.6 times faster
+    (dict(batch=4, heads_q=4, heads_kv=4, seqlen_q=1099, seqlen_kv=1099, head_dim=128, causal=0), 0),
+    (dict(batch=8, heads_q=8, heads_kv=8, seqlen_q=347, seqlen_kv=347, head_dim=128), 0),
+    (dict(batch=4, heads_q=28, heads_kv=4, seqlen_q=248, seqlen_kv=5228, head_dim=128, soft_cap=30.0), 0),
+    (dict(batch=4, heads_q=64, heads_kv=8, seqlen_q=1522, seqlen_kv=1522, doc_bounds=FAKE), 0),
+    (dict(batch=8, heads_q=2, heads_kv=2, seqlen_q=107, seqlen_kv=7443, head_dim=128, dtype=L.F32), 0),
+    (dict(batch=2, heads_q=32, heads_kv=8, seqlen_q=4096, seqlen_kv=4096, head_dim=128), 0),
+])
+def test_split_backward_is_preferred_where_it_is_faster(kw, split):
+    assert L.load().flexatt_bwd_prefers_split(problem(**kw)) == split
+
+
 def test_build_rejects_scratch_in_async_load_kernels():
     """The build guard reads the compiler's resource remarks: any kernel of a
     source with asm register loads that uses scratch fails the build."""
