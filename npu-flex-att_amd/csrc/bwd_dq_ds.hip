@@ -110,9 +110,9 @@ void bwd_dq_ds_kernel(BwdArgs a) {
   const int nkb = (p.Skv + kDsKB - 1) / kDsKB;
   const int nsb = (p.Skv + C::SB - 1) / C::SB;  // sub-blocks holding key rows
   constexpr int SPU = kDsKB / C::SB;            // sub-blocks per dS unit
-  // Slot c of wave v: 16 slots ordered (tile, head) so that the four slots
-  // of a wave lie in one aligned group of four query tiles (one causal band
-  // end).
+  // Slot c of wave v: the workgroup's SLOTS slots ordered (tile, head), NSL
+  // consecutive ones to a wave, so that a wave's slots lie in one aligned group
+  // of four query tiles (one causal band end).
   auto slot_of = [&](int v, int c, int& hq, int& t) {
     const int k = v * C::NSL + c;
     hq = hk * p.G + hg * nh + k % nh;

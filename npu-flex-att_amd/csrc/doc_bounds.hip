@@ -20,9 +20,9 @@ namespace {
 constexpr int kThreads = 1024, kPer = 8;
 constexpr int kWaves = kThreads / 64;
 
-// Inclusive scan over the workgroup of one int per thread, and the exclusive
-// value of this thread combined with `carry`.  DIR +1: max over the threads
-// before this one; -1: min over the threads after it.
+// Exclusive scan over the workgroup of one int per thread.  DIR +1: max over
+// the threads before this one; -1: min over the threads after it; `none` where
+// there is no such thread.
 template <int DIR>
 __device__ __forceinline__ int scan_exclusive(int v, int none, int* tot) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -52,7 +52,6 @@ __global__ __launch_bounds__(kThreads) void doc_bounds_kernel(const I* ids, int 
   bounds += (int64_t)blockIdx.x * S * 2;
   constexpr int CH = kThreads * kPer;
   const int nch = (S - 1) / CH + 1;
-  // whether position i (0 < i < S) starts a document
   I id[kPer + 1];  // ids of positions p0 - 1 .. p0 + kPer - 1 (clamped into the row)
   auto load = [&](int64_t p0) {
 #pragma unroll

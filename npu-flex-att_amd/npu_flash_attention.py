@@ -62,13 +62,14 @@ _DTYPES = {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _li
 decode_enabled = True
 # The backward stages dS through a workspace (flexatt_bwd_ws) whenever the
 # library supports it for the problem (fp16/bf16 at head_dim 64, 128 and 256;
-# fp32 at every head_dim) and reports that staging pays (below).  Set to
-# False to run the recomputing dQ kernel (flexatt_bwd).
+# fp32 at every head_dim) and reports that staging pays (below); small
+# problems take flexatt_bwd_split instead where it reports that this is faster.
+# Set to False to run the recomputing dQ kernel (flexatt_bwd).
 ds_staging_enabled = True
 # Stage only where flexatt_bwd_prefers_staging reports that staging pays:
 # not at head_dim 64 fp16/bf16 without soft-cap or interval/block masks,
 # where the recomputing backward measured 2-15% faster.  False: stage
-# wherever the staged range covers the problem.
+# wherever the staged range covers the problem, and never split.
 ds_staging_auto = True
 # Byte budget of that workspace for one backward call.  The whole dS band
 # (about one byte per attended (query row, key) pair of each query head for
