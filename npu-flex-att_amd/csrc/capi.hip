@@ -289,6 +289,11 @@ int cu_count() {
   return n;
 }
 
+int cus() {  // 256 if unknown
+  const int n = cu_count();
+  return n > 0 ? n : 256;
+}
+
 // Attended (query row, key) pairs of one head under the causal and window
 // masks (interval masks, whose bounds are on the device, not counted).
 int64_t attended_pairs(const flexatt_problem* p) {
@@ -339,7 +344,7 @@ int64_t attended_pairs(const flexatt_problem* p) {
 // the gain stays.  D = 256 loses its 1 us at one or two tiles of keys (S=42 8.7 against 10.1).
 int split_waves(const flexatt_problem* p) {
   if (p->block_map || !kSplit[p->dtype][head_index(p->head_dim)]) return 0;
-  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  const int64_t ncu = cus();
   const int64_t G = p->heads_q / p->heads_kv, groups = (int64_t)p->batch * p->heads_kv;
   const int64_t wgs = groups * ((G * p->seqlen_q + 31) / 32);
   int64_t keys = p->causal && p->seqlen_q < p->seqlen_kv ? p->seqlen_q : p->seqlen_kv;  // the longest row's
@@ -356,14 +361,14 @@ int split_waves(const flexatt_problem* p) {
     const double rows = p->seqlen_q <= 128 ? 0.6 : 1.0;  // the regular workgroup then runs one wave a SIMD
     return 5 + (c > w ? c : w) < 6 + rows * other[d] * chain ? 4 : 0;
   }
-  if (p->head_dim == 256) return wgs <= cus && chain > 2 ? 4 : 0;
+  if (p->head_dim == 256) return wgs <= ncu && chain > 2 ? 4 : 0;
   // (an eighth above the measured points, whose causal pairs are just over half)
-  const int64_t load = 8 * units / (cus * chain);  // in eighths
+  const int64_t load = 8 * units / (ncu * chain);  // in eighths
   if (load > (p->head_dim == 128 ? 18 : 36)) return 0;
   constexpr double pair[3] = {0.3, 0.5, 0.85}, wg[3] = {2.5, 3.7, 9.2};
   if ((pair[head_index(p->head_dim)] * units + wg[head_index(p->head_dim)] * wgs) / 1024 > 2 + 0.6 * chain) return 0;
-  if (p->head_dim == 128) return wgs <= cus && chain >= 64 && load <= 9 ? 8 : 4;
-  return wgs <= cus && chain >= 32 ? 8 : 4;
+  if (p->head_dim == 128) return wgs <= ncu && chain >= 64 && load <= 9 ? 8 : 4;
+  return wgs <= ncu && chain >= 32 ? 8 : 4;
 }
 
 int bwd_common(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
@@ -716,34 +721,41 @@ int64_t longest_walk(const flexatt_problem* p) {
 
 // Workgroups that share the query tiles of one KV block in the staged dK/dV
 // launch (fp16/bf16).  The launch lasts as long as its longest block, or as the
-// work per CU where that is longer; parts divide the first and cost their fp32 sums,
-// written and read at about 5.5 TB/s, and their launch.  Estimates in us, fitted to
-// 940 shapes (450 without documents: H = 1 .. 128, G = 1 .. 8, 64 .. 8000 positions, causal,
-// windowed and not; 490 with them): `tile` per 32-row query tile of the longest block, `work`
-// per tile and CU, `start` per 1024 workgroups, `sums` for their launch.  Of those shapes 7 without and 27 with
-// documents are more than 5% slower than one part; a rule that counted blocks
-// against CUs had 44 and 77.  Backward, parts 1 / 2 / 3 / 4, us, D = 128 causal: Hq=32
-// Hkv=8 S=4096 604 / 501 / 515 / 523, S=3000 429 / 333 / 318 / 331, S=2048 295 / 218 / 194 /
-// 194; documents of 100 on average S=3000 90 / 98 / 111, of 2000 310 / - / 226; Hq=Hkv=16 S=2048 of
-// 200 53 / 76 (G = 1: short walks, the same sums); D = 64 with half the blocks masked S=4096 416 / 311 / 285 /
-// 272; D = 256 Hq=16 S=1000 141 / 102 / 97 / 101.
+// work per CU where that is longer; parts divide the first (blocks of equal length
+// run in whole rounds) and cost their fp32 sums, written and read at about 5.5 TB/s,
+// and one more launch.  Estimates in us, fitted to 940 shapes (450 without documents: H = 1 ..
+// 128, G = 1 .. 8, 64 .. 8000 positions, causal, windowed and not; 490 with them): `tile` per
+// 32-row query tile of the longest block, `work` per tile and CU, `start` per 1024
+// workgroups, `sums` for the launch.  Under interval and block masks, whose walks may be
+// far shorter, parts have to gain a fifth of the walk besides: bf16 Hq=32 Hkv=8 S=7034 D=128,
+// parts 1 / 2, documents of 125 on average 186 / 231, 700 331 / 332, 2000 618 / 595.  Of 905 shapes it
+// was not fitted to, 19 are more than 5% slower than one part; a rule that counted blocks
+// against CUs had 144.  Backward, parts 1 / 2 / 3 / 4, D = 128 causal: Hq=32 Hkv=8 S=4096
+// 604 / 501 / 515 / 523, S=3000 429 / 333 / 318 / 331, S=2048 295 / 218 / 194 / 194; documents of
+// 2000 S=3000 310 / - / 226; Hq=Hkv=16 S=2048 of 200 53 / 76 (G = 1: short walks, the same sums);
+// D = 64 with half the blocks masked S=4096 416 / 311 / 285 / 272; D = 256 Hq=16 S=1000 141 / 102 / 97
+// / 101, non-causal Hq=14 Hkv=2 S=3561 (112 items on 256 CUs) - / 661 / 809.
 int staged_parts(const flexatt_problem* p) {
   if (!is_16bit(p) || p->head_dim == 32) return 1;
   const int d = head_index(p->head_dim);
   constexpr double tile[4] = {0, 0.91, 0.78, 0.94}, work[4] = {0, 0.92, 1.08, 1.0};
   constexpr double start[4] = {0, 0, 5.5, 5.0}, sums[4] = {0, 2.5, 0.7, 2.5};
-  const double cus = cu_count() > 0 ? cu_count() : 256, slots = p->head_dim == 64 ? 2 * cus : cus;
+  const double slots = p->head_dim == 64 ? 2 * cus() : cus();
   const int passes = p->head_dim == 256 ? 2 : 1;
   const int64_t nkb = (p->seqlen_kv + kDsKB - 1) / kDsKB, blocks = (int64_t)p->batch * p->heads_kv * nkb * passes;
+  const int64_t units = ds_units_per_head(p), walk = longest_walk(p);
   const double share = mask_share(p), cap = p->soft_cap > 0.f ? 1.2 : 1.0;
-  const double longest = tile[d] * cap * share * longest_walk(p) * (p->heads_q / p->heads_kv);
-  const double even = work[d] * cap * share * share * passes * p->batch * p->heads_q * ds_units_per_head(p) / slots;
+  const double longest = tile[d] * cap * share * walk * (p->heads_q / p->heads_kv);
+  const double even = work[d] * cap * share * share * passes * p->batch * p->heads_q * units / slots;
+  const bool equal = !has_masks(p) && units > 0.8 * nkb * walk;
+  const double margin = (has_masks(p) ? 0.2 : 0.01) * longest;
   const int64_t most = (p->seqlen_q + 4 * kDsQT - 1) / (4 * kDsQT);  // at least about four query tiles each
   double best = 1e30;
   int parts = 1;
   for (int n = 1; n <= 4 && n <= most; ++n) {
-    const double busy = even + start[d] * n * blocks / 1024, one = longest / n;
-    const double est = (one > busy ? one : busy) + (n > 1 ? sums[d] + 0.01 * longest + 0.36e-6 * part_bytes(p, n) : 0.0);
+    const double one = longest / n * (equal ? ceil(n * blocks / slots) : 1.0);
+    const double busy = even + start[d] * n * blocks / 1024;
+    const double est = (one > busy ? one : busy) + (n > 1 ? sums[d] + margin + 0.36e-6 * part_bytes(p, n) : 0.0);
     if (est < best) {
       best = est;
       parts = n;
@@ -761,102 +773,138 @@ bool bwd_split_applies(const flexatt_problem* p) {
   return kBwdSplit[p->dtype][head_index(p->head_dim)] && !p->block_map;
 }
 // The split backward's plan, and whether it beats the staged / recomputing
-// backward, from estimates in us fitted to graph replays of 950 shapes without documents
-// (H = 1 .. 128, G = 1 .. 8, 64 .. 8000 positions, B = 1 .. 8, causal, windowed and not).
-// A workgroup's time is its longest chain of 32 x 32 tiles (D = 128: 1.9 us a tile
-// and wave; 64: 1.45, 1.7 with eight waves, two to a SIMD; 32: 0.8) until the chip is full;
-// then the chip's time is `unit` per 1024 tile pairs and `wg` per 1024
-// workgroups.  The other backward's (BwdOtherCost) is its longest dK/dV walk, divided by
-// staged_parts, or the work per CU, and its longest dQ chain or the work; interval masks
-// count for mask_share.  Taken at 10% less.  Of 1550 shapes that neither this nor staged_parts was
-// fitted to, 19 are more than 5% slower than the other backward without parts, the worst 1.4
-// times; constants fitted to 56 shapes, without the work on the other side, had 106.
+// backward, from estimates in us fitted to graph replays of 3100 shapes without documents
+// (H = 1 .. 128, G = 1 .. 8, 64 .. 8000 positions, B = 1 .. 8, causal, windowed and not), rms 7 to
+// 13% a side, 20% at D = 32.
+// A split workgroup's time is its longest chain of 32 x 32 tiles until the chip is full; then the
+// chip's time is `unit` per 1024 tile pairs and `wg` per 1024 workgroups.  The other backward's
+// (BwdOtherCost) is its longest dK/dV walk, divided by staged_parts, or the work per CU, and its
+// longest dQ chain or the work; interval masks count for mask_share on both sides.  Of 890 other
+// shapes, a third of them with documents, 3 are more than 5% slower than the other backward
+// without parts, the worst 1.15 times; constants fitted to 56 shapes, without the work on the
+// other side, had 22.
 // Measured, other -> split (waves x splits): D = 64 H=2 S=2048 causal 75 -> 20
 // (8 x 1), Hq=8 Hkv=2 S=2048 193 -> 41 (8 x 2); D = 128 Hq=8 Hkv=2 S=1000 155
 // -> 34 (4 x 4), S=2048 286 -> 74 (4 x 2); past the crossover: Hq=32 Hkv=8 B=2 S=2048 D=128
 // 326 -> 472; D = 128 B=4 H=4 S=1099 73 -> 92, B=8 Hq=8 Hkv=8 S=347 causal 39 -> 51; D = 64 B=4
 // Hq=64 Hkv=8 S=1522 documents of 1000 on average 425 -> 533.
-struct BwdSplitPlan {
-  bool faster;
-  int nsplit, nw;
-  size_t bytes;
-};
-// fp32 (four waves; 250 of the shapes): D = 128 10 us a tile and wave, 19.5 us per 1024
-// pairs.  Other -> split: Hq=8 Hkv=2 S=1000 D=128 1264 -> 108 (4 x 4), H=2 S=2048 D=64 480
-// -> 93 (4 x 1); past the crossover: D = 128 B=8 H=2 Sq=107 Skv=7443 causal 71 -> 112.
+// fp32 (four waves; 740 of the shapes): Hq=8 Hkv=2 S=1000 D=128 1264 -> 108 (4 x 4), H=2 S=2048
+// D=64 480 -> 93 (4 x 1); past the crossover: D = 128 B=8 H=2 Sq=107 Skv=7443 causal 71 -> 112.
 struct BwdSplitCost {
   double tile4, tile8, base4, base8, unit, wg4, wg8;
 };
-constexpr BwdSplitCost kBwdSplitCost[2][3] = {
+// Which waves and splits (fitted to 86 shapes' choices) ...
+constexpr BwdSplitCost kBwdSplitPick[2][3] = {
     {{0.8, 1.0, 6.0, 7.0, 1.0, 5.0, 10.0},     // fp16/bf16, D = 32
-     {1.45, 1.7, 7.5, 8.0, 1.5, 9.0, 16.0},    // 64
-     {1.9, 0.0, 9.5, 0.0, 3.0, 22.0, 0.0}},    // 128 (four waves only)
+     {1.2, 1.4, 7.0, 8.5, 1.4, 8.0, 14.0},     // 64
+     {1.6, 0.0, 9.0, 0.0, 2.8, 20.0, 0.0}},    // 128 (four waves only)
     {{3.5, 0.0, 7.0, 0.0, 5.5, 8.0, 0.0},      // fp32, D = 32
      {5.7, 0.0, 8.0, 0.0, 9.0, 8.0, 0.0},      // 64
-     {10.3, 0.0, 13.0, 0.0, 19.5, 44.0, 0.0}}, // 128
+     {10.0, 0.0, 10.0, 0.0, 19.5, 10.0, 0.0}}, // 128
 };
-// The other backward: us around its kernels, per 32-row query tile of the longest dK/dV walk and per tile and CU of all,
-// per 32-key tile of the longest dQ chain and per 1024 tile pairs (0: the chain alone decided the fit).
-struct BwdOtherCost {
-  double base, kv, kv_work, q, q_work;
+// ... and how long they take (fitted to the 3100 shapes' times; rows as above).
+constexpr BwdSplitCost kBwdSplitTime[2][3] = {
+    {{1.15, 1.34, 6.6, 6.5, 1.07, 4.7, 9.3},
+     {1.45, 1.62, 7.5, 8.35, 1.52, 8.8, 15.3},
+     {1.88, 0.0, 9.3, 0.0, 3.05, 21.7, 0.0}},
+    {{4.4, 0.0, 7.0, 0.0, 4.8, 8.0, 0.0},
+     {6.7, 0.0, 8.5, 0.0, 8.5, 19.0, 0.0},
+     {10.7, 0.0, 13.0, 0.0, 18.8, 43.0, 0.0}},
 };
-BwdOtherCost bwd_other_cost(const flexatt_problem* p, bool staged) {
-  const int d = head_index(p->head_dim);
-  constexpr BwdOtherCost f32[3] = {{10.0, 3.3, 0.0, 1.2, 0.0}, {10.0, 5.3, 0.0, 1.9, 0.0}, {6.8, 8.1, 0.0, 5.1, 8.35}};
-  constexpr BwdOtherCost half[3] = {{16.0, 0.65, 0.0, 0.6, 0.0}, {15.2, 0.69, 1.52, 0.33, 0.53}, {20.7, 0.94, 1.12, 0.46, 0.79}};
-  constexpr BwdOtherCost half64_staged = {17.0, 1.11, 1.4, 0.15, 1.06};
-  return p->dtype == FLEXATT_F32 ? f32[d] : d == 1 && staged ? half64_staged : half[d];
-}
-BwdSplitPlan bwd_split_plan(const flexatt_problem* p) {
-  const bool f32 = p->dtype == FLEXATT_F32;
-  const BwdSplitCost& c = kBwdSplitCost[f32][head_index(p->head_dim)];
-  const bool cap = p->soft_cap > 0.f;
-  const double G = p->heads_q / p->heads_kv, groups = (double)p->batch * p->heads_kv, share = mask_share(p);
-  const int64_t nqt = (p->seqlen_q + 31) / 32, nkt = (p->seqlen_kv + 31) / 32;
-  int64_t lq = nqt, lk = nkt;  // longest streams: query tiles of a KV item, key tiles of a Q item
-  if (p->causal && nqt < lk) lk = nqt;
+// What both need of a problem.
+struct BwdStreams {
+  double G, groups, units, part;  // units: 1024 tile pairs; part: bytes of one split's sums
+  int64_t lq, lk, nkt, nrt;       // longest streams: query tiles of a KV item, key tiles of a Q item; tiles of each
+};
+BwdStreams bwd_streams(const flexatt_problem* p) {
+  BwdStreams s;
+  s.G = p->heads_q / p->heads_kv;
+  s.groups = (double)p->batch * p->heads_kv;
+  s.lq = (p->seqlen_q + 31) / 32;
+  s.nkt = s.lk = (p->seqlen_kv + 31) / 32;
+  if (p->causal && s.lq < s.lk) s.lk = s.lq;
   if (p->sliding_window > 0 && p->causal) {
     const int64_t l = p->sliding_window / 32 + 2;
-    if (l < lq) lq = l;
-    if (l < lk) lk = l;
+    if (l < s.lq) s.lq = l;
+    if (l < s.lk) s.lk = l;
   }
-  const double units = share * share * groups * G * (double)attended_pairs(p) / (32.0 * 32 * 1024);
-  const int64_t nrt = ((int64_t)(p->heads_q / p->heads_kv) * p->seqlen_q + 31) / 32;
-  const double part = 2.0 * sizeof(float) * groups * p->seqlen_kv * p->head_dim;  // bytes of one split's sums
+  s.nrt = ((int64_t)(p->heads_q / p->heads_kv) * p->seqlen_q + 31) / 32;
+  s.units = s.groups * s.G * (double)attended_pairs(p) / (32.0 * 32 * 1024);
+  s.part = (double)part_bytes(p, 1);
+  return s;
+}
+double bwd_split_us(const BwdSplitCost& c, const BwdStreams& s, bool cap, double share, int nw, int ns) {
+  const double t = nw == 8 ? c.tile8 : c.tile4, base = nw == 8 ? c.base8 : c.base4;
+  const double wgs = s.groups * (double)(s.nkt * ns + s.nrt) / 1024;
+  const double chain = t * share * (s.G * s.lq / ns > s.lk ? s.G * s.lq / ns : s.lk) / nw;
+  const double work = c.unit * (cap ? 1.25 : 1.0) * share * share * s.units + (nw == 8 ? c.wg8 : c.wg4) * wgs;
+  // the sums written and read back at about 8 TB/s (they stay in cache), and one more launch
+  return base + (chain > work ? chain : work) + (ns > 1 ? 4 + 0.25e-6 * ns * s.part : 0);
+}
+struct BwdSplitPlan {
+  int nsplit, nw;
+  size_t bytes;
+};
+BwdSplitPlan bwd_split_pick(const flexatt_problem* p, const BwdStreams& s) {
+  const bool f32 = p->dtype == FLEXATT_F32, cap = p->soft_cap > 0.f;
   double best = 1e30;
-  BwdSplitPlan r{false, 1, 4, 0};
+  BwdSplitPlan r{1, 4, 0};
   for (int nw = 4; nw <= (p->head_dim < 128 && !f32 ? 8 : 4); nw += 4)
     for (int ns = 1; ns <= 8; ns *= 2) {
-      const double t = nw == 8 ? c.tile8 : c.tile4, base = nw == 8 ? c.base8 : c.base4;
-      const double wgs = groups * (double)(nkt * ns + nrt) / 1024;
-      const double chain = t * share * (G * lq / ns > lk ? G * lq / ns : lk) / nw;
-      const double work = c.unit * (cap ? 1.25 : 1.0) * units + (nw == 8 ? c.wg8 : c.wg4) * wgs;
-      // the sums written and read back at about 7 TB/s (they stay in cache), and one more launch
-      const double est = base + (chain > work ? chain : work) + (ns > 1 ? 4 + 0.3e-6 * ns * part : 0);
+      const double est = bwd_split_us(kBwdSplitPick[f32][head_index(p->head_dim)], s, cap, 1.0, nw, ns);
       if (est < best) {
         best = est;
         r.nsplit = ns;
         r.nw = nw;
       }
     }
+  if (r.nsplit > 1) r.bytes = part_bytes(p, r.nsplit);
+  return r;
+}
+BwdSplitPlan bwd_split_plan(const flexatt_problem* p) { return bwd_split_pick(p, bwd_streams(p)); }
+
+// The other backward: us around its kernels, per 32-row query tile of the longest dK/dV walk and
+// per tile and CU of all, per 32-key tile of the longest dQ chain and per 1024 tile pairs, and
+// per 1024 query tiles of 32 rows (Delta and the ends of the dQ workgroups).
+struct BwdOtherCost {
+  double base, kv, kv_work, q, q_work, rows;
+};
+BwdOtherCost bwd_other_cost(const flexatt_problem* p, bool staged) {
+  const int d = head_index(p->head_dim);
+  constexpr BwdOtherCost f32[3] = {{4.8, 3.2, 3.7, 2.0, 1.5, 3.4},      // D = 32
+                                   {5.4, 4.85, 11.5, 2.55, 1.8, 5.9},   // 64
+                                   {2.5, 8.1, 8.7, 5.0, 5.3, 9.3}};     // 128
+  constexpr BwdOtherCost half[3] = {{18.5, 0.9, 0.72, 0.46, 0.12, 9.9},   // D = 32
+                                    {14.0, 0.64, 1.23, 0.36, 0.5, 7.6},   // 64, recomputing
+                                    {19.5, 0.85, 1.4, 0.48, 0.28, 7.8}};  // 128
+  constexpr BwdOtherCost half64_staged = {13.9, 1.03, 0.96, 0.42, 0.99, 5.25};
+  return p->dtype == FLEXATT_F32 ? f32[d] : d == 1 && staged ? half64_staged : half[d];
+}
+bool bwd_split_faster(const flexatt_problem* p) {
+  const BwdStreams s = bwd_streams(p);
+  const BwdSplitPlan plan = bwd_split_pick(p, s);
+  const bool cap = p->soft_cap > 0.f;
+  const double share = mask_share(p);
+  const BwdSplitCost& c = kBwdSplitTime[p->dtype == FLEXATT_F32][head_index(p->head_dim)];
+  const double split = bwd_split_us(c, s, cap, share, plan.nw, plan.nsplit);
   // the staged backward where it is preferred, its dK/dV streams shared by parts
   const bool staged = flexatt_bwd_prefers_staging(p);
   const int np = staged ? staged_parts(p) : 1;
   const BwdOtherCost o = bwd_other_cost(p, staged);
-  const double cus = cu_count() > 0 ? cu_count() : 256, slots = p->head_dim == 64 ? 2 * cus : cus;
-  const double walk = o.kv * share * G * longest_walk(p) / np;
+  const double walk = o.kv * share * s.G * longest_walk(p) / np;
+  const double slots = p->head_dim == 64 ? 2 * cus() : cus();
   const double even = o.kv_work * share * share * p->batch * p->heads_q * ds_units_per_head(p) / slots;
-  const double dq = o.q * share * lk, dq_even = o.q_work * units;
-  const double other = o.base + (cap ? 1.2 : 1.0) * (walk > even ? walk : even) + (dq > dq_even ? dq : dq_even) +
-                       (np > 1 ? 3 + 0.38e-6 * np * part : 0.0);
-  r.faster = best < 0.9 * other;
-  if (r.nsplit > 1) r.bytes = (size_t)(part * r.nsplit);
-  return r;
+  const double dq = o.q * share * s.lk, dq_even = o.q_work * share * share * s.units;
+  const double rows = o.rows * p->batch * p->heads_q * ((p->seqlen_q + 31) / 32) / 1024;
+  const double sums = np > 1 ? 3 + 0.38e-6 * part_bytes(p, np) : 0.0;
+  const double other = o.base + (cap ? 1.2 : 1.0) * (walk > even ? walk : even) +
+                       (dq > dq_even ? dq : dq_even) + rows + sums;
+  return split < 0.97 * other;
 }
 }  // namespace
 
 int flexatt_bwd_prefers_split(const flexatt_problem* p) {
-  return check_problem(p) == FLEXATT_OK && bwd_split_applies(p) && bwd_split_plan(p).faster;
+  return check_problem(p) == FLEXATT_OK && bwd_split_applies(p) && bwd_split_faster(p);
 }
 
 size_t flexatt_bwd_split_workspace(const flexatt_problem* p) {

@@ -480,12 +480,12 @@ def _backward_path(lib, p, device=None):
     the library prefers it and the sums it adds fit ``ds_workspace_limit``,
     else flexatt_bwd_ws, or with 0 bytes flexatt_bwd."""
     if ds_staging_enabled and ds_staging_auto and lib.flexatt_bwd_prefers_split(p):
-        ws_bytes = int(lib.flexatt_bwd_split_workspace(p))
-        if ws_bytes <= _workspace_budget(0):
+        ws_bytes = lib.flexatt_bwd_split_workspace(p)
+        if ws_bytes == 0 or ws_bytes <= _workspace_budget(0):
             return True, ws_bytes
     ws_bytes = _staged_workspace_bytes(lib, p, device)
     if ws_bytes and ws_bytes == lib.flexatt_bwd_workspace(p):
-        parts = int(lib.flexatt_bwd_ws_parts_bytes(p))  # whole band: dK/dV may share its blocks' streams
+        parts = lib.flexatt_bwd_ws_parts_bytes(p)  # whole band: dK/dV may share its blocks' streams
         if ws_bytes + parts <= _workspace_budget(0):
             ws_bytes += parts
     return False, ws_bytes
