@@ -333,15 +333,19 @@ int64_t attended_pairs(const flexatt_problem* p) {
 // S=4096 non-causal 1126 -> 753; D = 64 H=2 S=2048 318 -> 55; D = 32 H=8 S=2048 204
 // -> 43.  The estimate of a full chip (5.9 us per 1024 pairs at D = 128, the
 // regular kernel 4.5) keeps large problems on the regular kernel.
-// Many row tiles of few keys: each 32-row workgroup costs its launch, its Q rows
-// and its combine, `wg` us per 1024 of them besides `pair` per 1024 tile pairs,
-// which the regular kernel's one chain (0.6 us a tile, and 2 us more around it) must
-// outlast.  Fitted to 1700 shapes, 33 .. 5000 positions, B = 1 .. 8, windowed, causal
-// and not; without this term 5% of them were slower than the regular kernel: bf16
-// D = 128 B=8 Hq=32 Hkv=8 S=143 causal 11.9 (regular) against 18.0, window 32 Hq=32 Hkv=8
-// Sq=2286 Skv=72 16.0 against 23.4; D = 64 B=4 Hq=128 Hkv=16 S=144 causal 11.4 against 15.3;
-// fp32 D = 128 B=4 Hq=56 Hkv=8 S=183 73 against 108; with it none of 1300 others by 8%, and 97% of
-// the gain stays.  D = 256 loses its 1 us at one or two tiles of keys (S=42 8.7 against 10.1).
+// Many row tiles of few keys: each 32-row workgroup costs its launch, its Q rows and its combine
+// besides its tile pairs (`wg` per 1024 of them, `pair` per 1024 pairs), against a regular
+// workgroup whose chain spans all its rows' keys (with a window, the window and those rows).
+// Estimates in us of both (FwdCost: split with four waves, regular), fitted to 1700 shapes, 33 ..
+// 5000 positions, B = 1 .. 8, windowed, causal and not, where the line above alone left 5% of the
+// calls more than 5% slower than the regular kernel: bf16 D = 128 B=8 Hq=32 Hkv=8 S=143 causal 11.9
+// (regular) against 18.0, window 32 Hq=32 Hkv=8 Sq=2286 Skv=72 16.0 against 23.4; D = 64 B=4 Hq=128
+// Hkv=16 S=144 causal 11.4 against 15.3; fp32 D = 128 B=4 Hq=56 Hkv=8 S=183 73 against 108.  Of 1184
+// other shapes 2 are now, of 28.
+// D = 256 loses its 1 us at one or two tiles of keys (S=42 8.7 against 10.1).
+struct FwdCost {
+  double base, tile, pair, wg, reg_base, reg_tile, reg_pair, reg_wg;
+};
 int split_waves(const flexatt_problem* p) {
   if (p->block_map || !kSplit[p->dtype][head_index(p->head_dim)]) return 0;
   const int64_t ncu = cus();
@@ -355,7 +359,8 @@ int split_waves(const flexatt_problem* p) {
   const int64_t chain = (keys + 31) / 32;
   const int64_t units = groups * G * attended_pairs(p) / (32 * 32);
   if (p->dtype == FLEXATT_F32) {
-    constexpr double tile[3] = {1.9, 3.2, 5.85}, unit[3] = {1.7, 2.9, 5.9}, other[3] = {3.2, 5.0, 8.4}, wg[3] = {5, 15, 32};
+    constexpr double tile[3] = {1.9, 3.2, 5.85}, unit[3] = {1.7, 2.9, 5.9}, other[3] = {3.2, 5.0, 8.4};
+    constexpr double wg[3] = {5, 15, 32};
     const int d = head_index(p->head_dim);
     const double c = tile[d] * chain / 4, w = (unit[d] * units + wg[d] * wgs) / 1024;
     const double rows = p->seqlen_q <= 128 ? 0.6 : 1.0;  // the regular workgroup then runs one wave a SIMD
@@ -365,10 +370,21 @@ int split_waves(const flexatt_problem* p) {
   // (an eighth above the measured points, whose causal pairs are just over half)
   const int64_t load = 8 * units / (ncu * chain);  // in eighths
   if (load > (p->head_dim == 128 ? 18 : 36)) return 0;
-  constexpr double pair[3] = {0.3, 0.5, 0.85}, wg[3] = {2.5, 3.7, 9.2};
-  if ((pair[head_index(p->head_dim)] * units + wg[head_index(p->head_dim)] * wgs) / 1024 > 2 + 0.6 * chain) return 0;
-  if (p->head_dim == 128) return wgs <= ncu && chain >= 64 && load <= 9 ? 8 : 4;
-  return wgs <= ncu && chain >= 32 ? 8 : 4;
+  if (wgs <= ncu && (p->head_dim == 128 ? chain >= 64 && load <= 9 : chain >= 32)) return 8;
+  constexpr FwdCost cost[3] = {{4.3, 0.54, 0.30, 2.5, 6.6, 0.43, 0.32, 2.1},   // D = 32
+                               {4.8, 0.72, 0.48, 3.7, 6.0, 0.60, 0.38, 2.5},   // 64
+                               {5.6, 1.02, 0.85, 9.2, 7.8, 0.70, 0.54, 4.7}};  // 128
+  const FwdCost& c = cost[head_index(p->head_dim)];
+  // the regular workgroup's chain: 256 rows, shared by up to 8 heads of a group
+  const int64_t low = G & -G, rows = 256 / (low < 8 ? low : 8);
+  int64_t reg_keys = p->causal && p->seqlen_q < p->seqlen_kv ? p->seqlen_q : p->seqlen_kv;
+  if (p->sliding_window > 0) {
+    const int64_t w = p->sliding_window + (p->causal ? (rows < p->seqlen_q ? rows : p->seqlen_q) : (int64_t)p->seqlen_kv);
+    if (w < reg_keys) reg_keys = w;
+  }
+  const double wait = c.tile * chain / 4, busy = (c.pair * units + c.wg * wgs) / 1024;
+  const double reg_wait = c.reg_tile * ((reg_keys + 31) / 32), reg_busy = (c.reg_pair * units + c.reg_wg * wgs) / 1024;
+  return c.base + (wait > busy ? wait : busy) < c.reg_base + (reg_wait > reg_busy ? reg_wait : reg_busy) ? 4 : 0;
 }
 
 int bwd_common(const flexatt_problem* p, const flexatt_tensor* q, const flexatt_tensor* k,
