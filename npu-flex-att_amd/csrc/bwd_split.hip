@@ -9,8 +9,8 @@
 // dS = P (dP - Delta) scale (1 - tanh^2), dV = P^T dO, dK = dS^T Q, dQ = dS K.
 // P and dS are rounded to the input dtype before their MFMAs, as the
 // reference does before tl.dot: dS with the scale in it at D = 32 and without it
-// above (the gradient is scaled instead), as the other backward kernels of each
-// head dim round it, so that fp16 has one range whatever the size selects.
+// above (the gradient is scaled instead), as the kernels that larger problems of
+// each head dim take round it, so that the size does not change fp16's range.
 //
 // Decomposition
 //  * Two kinds of items in one grid, so that neither waits for the other:
