@@ -206,7 +206,7 @@ int decode_run(const flexatt_problem* p, const DecodePlan& d, const flexatt_tens
   a.nsplit = d.nsplit;
   a.chunk = d.chunk;
   a.nw = nw;
-  a.nrt = 0;
+  a.nrt = a.plain = 0;
   const int64_t rows = (int64_t)p->batch * p->heads_q * p->seqlen_q;
   a.part_o = (float*)ws;
   a.part_lse = a.part_o + rows * d.nsplit * p->head_dim;

@@ -62,6 +62,7 @@ struct DecodeArgs {
   int chunk;   // 32-row KV tiles per workgroup (nsplit > 1)
   int nw;      // waves per workgroup with one split (4 or 8; D = 256: 4)
   int nrt;     // 32-row tiles of packed query rows per (b, hkv) (set by the launcher)
+  int plain;   // workgroups in plain order instead of by XCD (set by the launcher)
 };
 
 // Backward in one launch with the streams split over waves (bwd_split.hip).

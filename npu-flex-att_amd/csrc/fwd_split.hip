@@ -87,7 +87,7 @@ void fwd_split_kernel(DecodeArgs a) {
   const int s = blockIdx.x % a.nsplit;
   const int item = blockIdx.x / a.nsplit;
   int krt, bh;
-  if (a.nsplit > 1 || a.nrt == 1 || !xcd_lpt_item(item, a.nrt, p.B * p.Hkv, krt, bh)) {
+  if (a.plain || !xcd_lpt_item(item, a.nrt, p.B * p.Hkv, krt, bh)) {
     krt = item % a.nrt;
     bh = item / a.nrt;
   }
@@ -436,6 +436,7 @@ template <class T, int D>
 hipError_t launch_split(const DecodeArgs& a, hipStream_t st) {
   DecodeArgs x = a;
   x.nrt = (int)(((int64_t)a.p.G * a.p.Sq + 31) / 32);
+  x.plain = x.nsplit > 1 || x.nrt == 1;
   if constexpr (D == 256) {
     return launch_split<T, D, 4, 1>(x, st);
   } else {
